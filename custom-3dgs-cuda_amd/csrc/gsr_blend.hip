@@ -24,14 +24,21 @@
 // when none of its pixels is live; the tile stops when all are done.
 // Backward: the tile walks only entries [0, max n_contrib) of its list, back
 // to front (the reference walks all K entries and skips the tail per pixel),
-// and each wave skips entries beyond its own max n_contrib; each entry's nine
-// gradient sums are formed in the lane, summed across the wave (one
-// transposed permlane/DPP reduction) and across the waves through LDS, then
-// stored with plain stores into the (Gaussian, tile) pair's own gradient slot
+// and each wave skips entries beyond its own max n_contrib.  It takes its
+// entries four at a time: their decisions in straight-line code, their colours'
+// products with dL/dpixel by matrix instructions, and their nine gradient sums
+// over the wave through one transposition in LDS (see group_sums).  The two
+// waves' sums of an entry are added and stored with plain stores into the
+// (Gaussian, tile) pair's own gradient slot
 // (nine floats and a claim bit).  pair_grad_reduce_kernel adds each
 // Gaussian's claimed slots.  Float atomics are used only for list entries
 // that have no slot of their own: pairs outside the Gaussian's tile
 // rectangle, and a repeated id within one tile's list (caller-supplied lists).
+// Measured with a wave reduction per entry and so (same run): 229 and 213 us
+// (100k Gaussians, 1080p), 288 and 275 us (1M), 96 and 76 us (10k, 256x256);
+// VALU instructions per 1080p launch 1.38e8 and 1.09e8.  VALU issue takes 0.70
+// of the slots; the waves' dependent chains (LDS, exp, compares and their
+// masks) and the prologue's and batches' loads leave the rest.
 //
 // Work-groups take their tile from a launch order, longest estimated work
 // first (tile_order_kernel), so long tiles do not start last.
@@ -77,6 +84,22 @@ __device__ __forceinline__ Pixels<kPix> pixels_of(int tile, int tiles_x, int W, 
     return p;
 }
 
+// The backward's pixels: the same strips, a lane's two pixels in adjacent
+// rows 2 (l >> 4) + k, so that a quad of lanes holds four columns of two
+// adjacent rows (group_sums takes their moments).
+__device__ __forceinline__ Pixels<2> bwd_pixels_of(int tile, int tiles_x, int W, int H) {
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int tx = tile % tiles_x, ty = tile / tiles_x;
+    Pixels<2> p;
+    p.px = tx * kTileSize + (lane & 15);
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        p.py[k] = ty * kTileSize + wave * Layout<2>::kRows + 2 * (lane >> 4) + k;
+        p.in[k] = p.px < W && p.py[k] < H;
+    }
+    return p;
+}
+
 // Minimum over the pixel rectangle [x0, x1] x [y0, y1] of the quadratic form
 // q = A u^2 + 2 B u v + C v^2, (u, v) = (x - mx, y - my), for a positive
 // definite conic (A > 0, AC > B^2): 0 when the mean is inside, else the least
@@ -96,15 +119,19 @@ __device__ __forceinline__ float qmin_rect(float mx, float my, float A, float B,
     return best;
 }
 
-// Staged strip bits: bit w for wave w of the tile, and this flag for the
-// backward (opacity in [0, 0.99)).
-constexpr uint32_t kFastExpBit = 1u << 31;
+// Staged strip bits: bit w for wave w of the tile, and this flag for a plain
+// entry: a plain record (plain_record) whose quadratic form's |terms| sum to at
+// most kPlainTerms over the tile, so that exp's argument reduction holds and
+// gives 0 or a denormal far below the range, an alpha below 1/255 either way.
+constexpr uint32_t kPlainBit = 1u << 31;
+constexpr float kPlainTerms = 4e6f;
 
 // Bit w set: some pixel of strip w may reach alpha >= 1/255.  A strip is
 // culled when the least q over its rectangle, lowered by 1e-5 of the largest
 // sum of |terms| there (the fp32 rounding of the per-pixel q and of this
 // bound are each within ~1e-6 of that sum), still exceeds qthr.  Conics that
-// are not positive definite, and NaN anywhere, cull nothing.
+// are not positive definite, and NaN anywhere, cull nothing.  With kPlainBit
+// for a plain entry.
 template <int kPix>
 __device__ __forceinline__ uint32_t strip_bits(const BlendRec& r, int tile, int tiles_x) {
     constexpr uint32_t kAll = (1u << Layout<kPix>::kWaves) - 1u;
@@ -117,6 +144,7 @@ __device__ __forceinline__ uint32_t strip_bits(const BlendRec& r, int tile, int 
     const float x0 = (float)(tx * kTileSize), x1 = x0 + (float)(kTileSize - 1);
     const float dxm = fmaxf(fabsf(x0 - mx), fabsf(x1 - mx));
     uint32_t bits = 0;
+    float most = 0.0f;  // the largest sum of |terms| over the tile
 #pragma unroll 1
     for (int w = 0; w < Layout<kPix>::kWaves; ++w) {
         const float y0 = (float)(ty * kTileSize + w * Layout<kPix>::kRows);
@@ -126,8 +154,9 @@ __device__ __forceinline__ uint32_t strip_bits(const BlendRec& r, int tile, int 
         const float q = qmin_rect(mx, my, A, B, C, rA, rC, x0, x1, y0, y1) - 1e-5f * absq;
         const bool skip = q > thr;  // false for NaN
         bits |= skip ? 0u : (1u << w);
+        most = (absq <= most) ? most : absq;  // NaN stays
     }
-    return bits;
+    return bits | (r.c.w == kPlainRecord && most <= kPlainTerms ? kPlainBit : 0u);
 }
 
 // The record of list entry g, zeros for an id outside [0, n) (such entries are
@@ -142,30 +171,26 @@ __device__ __forceinline__ BlendRec load_record(const BlendRec* __restrict__ rec
     return r;
 }
 
-template <int kPix>
-__device__ __forceinline__ void stage_record(const BlendRec& r, bool ok, int g, int tile,
-                                             int tiles_x, float4* s_a, float4* s_b, float4* s_c,
-                                             uint32_t* s_bits, int* s_id, int slot) {
-    s_a[slot] = r.a;
-    s_b[slot] = r.b;
-    if (s_bits) s_c[slot] = r.c;
-    // bit 31: opacity in [0, 0.99), so alpha = opacity * G is never clamped
-    const uint32_t fast = (__float_as_uint(r.b.y) < __float_as_uint(kAlphaMax)) ? kFastExpBit : 0u;
-    const uint32_t bits = ok ? (strip_bits<kPix>(r, tile, tiles_x) | fast) : 0u;
-    if (s_bits)
-        s_bits[slot] = bits;
-    else  // in the record's unused fourth word
-        s_c[slot] = make_float4(r.c.x, r.c.y, r.c.z, __uint_as_float(bits));
-    if (s_id) s_id[slot] = ok ? g : -1;
-}
-
+// A staged entry: the record's a and b words, and of c the blue channel and the
+// strip bits (c.y is a.w / 2, exactly; qthr has served).
 template <int kPix>
 __device__ __forceinline__ void stage_entry(const BlendRec* __restrict__ recs, int g, int n,
                                             int tile, int tiles_x, float4* s_a, float4* s_b,
-                                            float4* s_c, uint32_t* s_bits, int* s_id,
-                                            int slot) {
-    stage_record<kPix>(load_record(recs, g, n), g >= 0 && g < n, g, tile, tiles_x, s_a, s_b, s_c,
-                       s_bits, s_id, slot);
+                                            float2* s_c, int* s_id, int slot) {
+    const BlendRec r = load_record(recs, g, n);
+    const bool ok = g >= 0 && g < n;
+    s_a[slot] = r.a;
+    s_b[slot] = r.b;
+    const uint32_t bits = ok ? strip_bits<kPix>(r, tile, tiles_x) : 0u;
+    s_c[slot] = make_float2(r.c.x, __uint_as_float(bits));
+    if (s_id) s_id[slot] = ok ? g : -1;
+}
+
+// The entry past a batch's last place, which fills up a backward group: its
+// opacity is 0, so no pixel blends it.
+__device__ __forceinline__ void stage_none(float4* s_a, float4* s_b, float2* s_c, int slot) {
+    s_a[slot] = s_b[slot] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    s_c[slot] = make_float2(0.0f, __uint_as_float(kPlainBit));
 }
 
 // Forward pixel state.  A pixel is done once a blend takes T below 1e-4
@@ -207,21 +232,61 @@ __device__ __forceinline__ void fwd_step(FwdPixel& p, bool on, float fx, float f
     p.last = blend ? contributor : p.last;
 }
 
+// fwd_step of the next kCount plain entries (kPlainBit) of `todo` in list order,
+// bit for bit: a plain entry's power is never positive, its alpha never clamped,
+// exp needs no range select, and one select of alpha serves the colours and T
+// (a weight of 0 adds nothing, T times 1 is T): 28 VALU per pixel and entry
+// instead of 35.  The alphas do not depend on T: all of the group's are formed
+// first, in straight-line code with independent chains, then blended in order.
+// Measured with a step per entry and so (same run): 140 and 123 us (100k
+// Gaussians, 1080p), 180 and 157 us (1M), 48 and 41 us (10k, 256x256).
+constexpr int kFwdGroup = 4;
+template <int kPix, int kCount>
+__device__ __forceinline__ void fwd_steps_plain(FwdPixel (&p)[kPix], float fx,
+                                                const float (&fy)[kPix], const float4* s_a,
+                                                const float4* s_b, const float2* s_c, int c0,
+                                                uint64_t& todo, int cbase) {
+    float alpha[kCount][kPix];
+    int at[kCount];
+#pragma unroll
+    for (int s = 0; s < kCount; ++s) {
+        at[s] = c0 + (int)__builtin_ctzll(todo);
+        todo &= todo - 1;
+        const float4 A = s_a[at[s]];
+        const float2 B = *reinterpret_cast<const float2*>(s_b + at[s]);
+        const float dx = fx - A.x;
+        const float adxdx = (A.z * dx) * dx, bdx = A.w * dx;  // blend_power's column terms
+#pragma unroll
+        for (int k = 0; k < kPix; ++k) {
+            const float dy = fy[k] - A.y;
+            const float power = __builtin_fmaf(B.x * dy, dy, __builtin_fmaf(bdx, dy, adxdx));
+            const float a = B.y * exp_core(power);
+            alpha[s][k] = (a < kAlphaMin) ? 0.0f : a;
+        }
+    }
+#pragma unroll
+    for (int s = 0; s < kCount; ++s) {
+        const float2 rg = *(reinterpret_cast<const float2*>(s_b + at[s]) + 1);
+        const float cb = s_c[at[s]].x;
+#pragma unroll
+        for (int k = 0; k < kPix; ++k) {
+            const float a = live(p[k]) ? alpha[s][k] : 0.0f;
+            const float w = a * p[k].T;
+            p[k].C0 = __builtin_fmaf(rg.x, w, p[k].C0);
+            p[k].C1 = __builtin_fmaf(rg.y, w, p[k].C1);
+            p[k].C2 = __builtin_fmaf(cb, w, p[k].C2);
+            p[k].T = p[k].T * (1.0f - a);
+            p[k].last = (a > 0.0f) ? cbase + at[s] : p[k].last;
+        }
+    }
+}
+
 template <int kPix>
 __device__ __forceinline__ bool any_live(const FwdPixel (&p)[kPix]) {
     bool l = false;
 #pragma unroll
     for (int k = 0; k < kPix; ++k) l |= live(p[k]);
     return l;
-}
-
-// A staged entry's strip bits as a wave-uniform (scalar) value: from the
-// separate array, or from the record's unused fourth word.
-__device__ __forceinline__ uint32_t uniform_bits(const uint32_t* s_bits, int j) {
-    return __builtin_amdgcn_readfirstlane(s_bits[j]);
-}
-__device__ __forceinline__ uint32_t uniform_bits(const float4& c) {
-    return __builtin_amdgcn_readfirstlane(__float_as_uint(c.w));
 }
 
 template <int kPix>
@@ -233,8 +298,7 @@ __global__ __launch_bounds__(Layout<kPix>::kThreads) void blend_fwd_kernel(
     constexpr int kBatch = Layout<kPix>::kBatch;
     __shared__ float4 s_a[kBatch];
     __shared__ float4 s_b[kBatch];
-    __shared__ float4 s_c[kBatch];
-    __shared__ uint32_t s_bits[kBatch];
+    __shared__ float2 s_c[kBatch];
     const int tile = order ? (int)order[blockIdx.x] : (int)blockIdx.x;
     // a launch order is a permutation of the tiles; nothing else is touched
     if ((unsigned)tile >= (unsigned)(tiles_x * ((H + kTileSize - 1) / kTileSize))) return;
@@ -242,13 +306,15 @@ __global__ __launch_bounds__(Layout<kPix>::kThreads) void blend_fwd_kernel(
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // scalar: uniform branches
     const uint32_t my_bit = 1u << wave;
     const Pixels<kPix> pp = pixels_of<kPix>(tile, tiles_x, W, H);
-    const float fx = (float)pp.px;
+    float fx = (float)pp.px;
+    asm volatile("" : "+v"(fx));
     float fy[kPix];
     FwdPixel p[kPix];
 #pragma unroll
     for (int k = 0; k < kPix; ++k) {
         fy[k] = (float)pp.py[k];
         p[k] = FwdPixel{pp.in[k] ? 1.0f : 0.0f, 0.0f, 0.0f, 0.0f, 0};
+        asm volatile("" : "+v"(fy[k]));  // kept as floats, not converted again per entry
     }
     int start, end;
     clamp_range(ranges[tile], m, start, end);
@@ -264,7 +330,7 @@ __global__ __launch_bounds__(Layout<kPix>::kThreads) void blend_fwd_kernel(
         const int g = next_id;
         __syncthreads();
         if (tid < cnt)
-            stage_entry<kPix>(recs, g, n, tile, tiles_x, s_a, s_b, s_c, s_bits, nullptr, tid);
+            stage_entry<kPix>(recs, g, n, tile, tiles_x, s_a, s_b, s_c, nullptr, tid);
         if (b0 + kBatch + tid < end) next_id = ids[b0 + kBatch + tid];
         __syncthreads();
         if (ballot(any_live(p)) != 0) {
@@ -275,23 +341,31 @@ __global__ __launch_bounds__(Layout<kPix>::kThreads) void blend_fwd_kernel(
             bool done = false;
             for (int c0 = 0; c0 < cnt && !done; c0 += kWave) {
                 const int e = c0 + lane;
-                uint64_t todo = ballot(e < cnt && (s_bits[min(e, kBatch - 1)] & my_bit) != 0u);
-                while (todo) {
-                    // the wave stops once no pixel is live, tested before each
-                    // entry with the same compares the step's skip uses
-                    if (ballot(any_live(p)) == 0) {
-                        done = true;
-                        break;
-                    }
-                    const int j = c0 + (int)__builtin_ctzll(todo);
-                    todo &= todo - 1;
-                    const float4 A = s_a[j];
-                    const float4 B = s_b[j];
-                    const float cb = s_c[j].x;
+                const uint32_t bits = e < cnt ? __float_as_uint(s_c[min(e, kBatch - 1)].y) : 0u;
+                uint64_t todo = ballot((bits & my_bit) != 0u);
+                const uint64_t plain = ballot((bits & kPlainBit) != 0u);
+                // the wave stops once no pixel is live, tested before each group
+                // or entry with the same compares the steps' skips use
+                if ((todo & ~plain) == 0) {
+                    int left = popc64(todo);
+                    for (; left >= kFwdGroup && ballot(any_live(p)) != 0; left -= kFwdGroup)
+                        fwd_steps_plain<kPix, kFwdGroup>(p, fx, fy, s_a, s_b, s_c, c0, todo,
+                                                         cbase);
+                    for (; left > 0 && ballot(any_live(p)) != 0; --left)
+                        fwd_steps_plain<kPix, 1>(p, fx, fy, s_a, s_b, s_c, c0, todo, cbase);
+                } else {
+                    while (todo && ballot(any_live(p)) != 0) {
+                        const int j = c0 + (int)__builtin_ctzll(todo);
+                        todo &= todo - 1;
+                        const float4 A = s_a[j];
+                        const float4 B = s_b[j];
+                        const float cb = s_c[j].x;
 #pragma unroll
-                    for (int k = 0; k < kPix; ++k)
-                        fwd_step(p[k], live(p[k]), fx, fy[k], A, B, cb, cbase + j);
+                        for (int k = 0; k < kPix; ++k)
+                            fwd_step(p[k], live(p[k]), fx, fy[k], A, B, cb, cbase + j);
+                    }
                 }
+                done = todo != 0;
             }
         }
         if (__syncthreads_and(!any_live(p))) break;
@@ -328,69 +402,51 @@ struct BwdTerms {
 
 // One pixel's decision for one list entry (rasterize_backward.cu:117-140):
 // G = exp(power), alpha = min(0.99, opacity G), and whether the entry blends
-// (within n_contrib, power <= 0, alpha >= 1/255) and passes gradient through
-// the clamp.  ae = alpha if it blends, else 0; ag = alpha if it also passes
-// gradient (then alpha = opacity G unclamped), else 0.
-struct BwdDecision {
-    float dy, power, alpha, ae, ag;
-    bool act;
-};
-
+// (within n_contrib, power <= 0, alpha >= 1/255).  ae = alpha if it blends,
+// else 0.  `within`: the lanes whose n_contrib the entry is within.  Each returns
+// the lanes that blend it.
+//
 // The forward's own evaluation: exp_blend and the same fp32 operations, so
-// every skip agrees with the forward bit for bit.
-__device__ __forceinline__ void decide_exact(BwdDecision& d, float o, int contributor, int last) {
-    const float araw = o * exp_blend(d.power);
-    d.alpha = fminf(kAlphaMax, araw);
-    d.act = (contributor <= last) & !(d.power > 0.0f) & !(d.alpha < kAlphaMin);
-    d.ae = d.act ? d.alpha : 0.0f;
-    d.ag = (d.act & (araw < kAlphaMax)) ? d.alpha : 0.0f;
+// every skip agrees with the forward bit for bit.  `clamped`: the lanes whose
+// alpha is clamped (no gradient through alpha).
+__device__ __forceinline__ uint64_t decide_exact(float power, float o, uint64_t within,
+                                                 float& ae, uint64_t& clamped) {
+    const float araw = o * exp_blend(power);
+    const float alpha = fminf(kAlphaMax, araw);
+    const uint64_t act =
+        within & ballot(!(power > 0.0f)) & ballot(!(alpha < kAlphaMin));
+    ae = __builtin_amdgcn_inverse_ballot_w64(act) ? alpha : 0.0f;
+    clamped = act & ~ballot(araw < kAlphaMax);
+    return act;
 }
 
-// For an entry with opacity in [0, 0.99): G from the hardware exp2, which is
-// within 1e-6 relative of exp_blend wherever alpha can reach 1/255 (power in
-// [-5.6, 0]), so the alpha >= 1/255 test agrees with the exact one unless
-// alpha lies within kNearAlpha of 1/255; alpha <= opacity < 0.99 is never
-// clamped.  Alpha at or above kAlphaMin + kNearAlpha passes the test, below
-// kAlphaMin - kNearAlpha fails it; the returned mask holds the lanes in
+// For a plain entry (kPlainBit: its power is never positive): G from the
+// hardware exp2, which is within 1e-6 relative of exp_blend wherever alpha can
+// reach 1/255 (power in [-5.6, 0]), so the alpha >= 1/255 test agrees with the
+// exact one unless alpha lies within kNearAlpha of 1/255; alpha <= opacity <
+// 0.99 is never clamped.  Alpha at or above kAlphaMin + kNearAlpha passes the
+// test, below kAlphaMin - kNearAlpha fails it; `near` holds the lanes in
 // neither case (near the threshold, or a NaN alpha), which need the exact
 // evaluation.  Two compares per pixel, each ballot a compare's own mask.
 constexpr float kNearAlpha = kAlphaMin * 2e-5f;
 constexpr float kAlphaLo = kAlphaMin - kNearAlpha, kAlphaHi = kAlphaMin + kNearAlpha;
-__device__ __forceinline__ uint64_t decide_fast(BwdDecision& d, float o, int contributor,
-                                                int last) {
-    d.alpha = o * __builtin_amdgcn_exp2f(d.power * 1.44269504088896341f);
-    const bool pass = d.alpha >= kAlphaHi;
-    d.act = (contributor <= last) & !(d.power > 0.0f) & pass;
-    d.ae = d.act ? d.alpha : 0.0f;
-    d.ag = d.ae;
-    return ballot(!(d.alpha < kAlphaLo)) & ~ballot(pass);
-}
-
-// The wave's decisions for one entry: the fast evaluation where the record
-// allows it, the exact one for the whole wave when any lane is near the
-// threshold.
-template <int kPix>
-__device__ __forceinline__ void decide_entry(BwdDecision (&d)[kPix], float o, bool fast,
-                                             int contributor, const BwdPixel (&p)[kPix]) {
-    bool exact = !fast;
-    if (!exact) {
-        uint64_t near = 0;
-#pragma unroll
-        for (int k = 0; k < kPix; ++k) near |= decide_fast(d[k], o, contributor, p[k].last);
-        exact = near != 0;
-    }
-    if (exact) {
-#pragma unroll
-        for (int k = 0; k < kPix; ++k) decide_exact(d[k], o, contributor, p[k].last);
-    }
+__device__ __forceinline__ uint64_t decide_fast(float power, float o, uint64_t within,
+                                                float& ae, uint64_t& near) {
+    const float alpha = o * __builtin_amdgcn_exp2f(power * 1.44269504088896341f);
+    const uint64_t pass = ballot(alpha >= kAlphaHi);
+    const uint64_t act = within & pass;
+    ae = __builtin_amdgcn_inverse_ballot_w64(act) ? alpha : 0.0f;
+    near |= ballot(!(alpha < kAlphaLo)) & ~pass;
+    return act;
 }
 
 // One pixel's gradient step for a decided entry (rasterize_backward.cu:
-// 141-198).  A skipped entry enters with ae = ag = 0, which leaves T (x / 1)
-// and accg unchanged and gives zero terms.  This arithmetic only has to meet
+// 141-198); cg is the entry's colour . dL/dpixel.  A skipped entry enters with ae = 0, which leaves T (x / 1) and
+// accg unchanged and gives zero terms.  dL/dpower is alpha T (colour .
+// dL/dpixel less what lies behind); the caller zeroes it where alpha is
+// clamped.  This arithmetic only has to meet
 // the fp32 gradient tolerance and may use fused multiply-adds.
-__device__ __forceinline__ BwdTerms bwd_update(BwdPixel& p, const BwdDecision& d,
-                                               const float4& B, float cb) {
+__device__ __forceinline__ BwdTerms bwd_update(BwdPixel& p, float ae, float cg) {
 #pragma clang fp contract(fast)
     BwdTerms t;
     // T / (1 - alpha) with 1 - alpha in [0.01, 1]: the reference's 1e-4 floor
@@ -406,13 +462,12 @@ __device__ __forceinline__ BwdTerms bwd_update(BwdPixel& p, const BwdDecision& d
     // error against float64, as did the forward's own alpha in place of the
     // fast one.  A skipped entry (alpha 0) leaves T unchanged: the reciprocal
     // of 1 is exact.
-    const float den = 1.0f - d.ae;
+    const float den = 1.0f - ae;
     const float Tb = p.T * __builtin_amdgcn_rcpf(den);
-    const float cg = B.z * p.g0 + B.w * p.g1 + cb * p.g2;
     const float diff = cg - p.accg;
-    t.aT = d.ae * Tb;
-    t.dpw = d.ag * (diff * Tb);
-    p.accg = __builtin_fmaf(d.ae, diff, p.accg);
+    t.aT = ae * Tb;
+    t.dpw = ae * (diff * Tb);
+    p.accg = __builtin_fmaf(ae, diff, p.accg);
     p.T = Tb;
     return t;
 }
@@ -435,26 +490,160 @@ __device__ __forceinline__ BwdPixel load_bwd_pixel(bool in, int px, int py, int 
     return p;
 }
 
-// Per (tile, entry) the wave sums nine values.  A lane's pixels share dx
-// (column lane & 15), so the reference's per-pixel mean and conic terms
-// (rasterize_backward.cu:163-176) follow from per-lane sums of dpw = dL/dpower:
-// S0 = sum dpw, P2 = sum dpw dy, P5 = sum dpw dy^2, with dx applied once the
-// lanes of a column are summed (wave_reduce_columns): P1 = sum dx S0,
-// Q1 = sum dx^2 S0, Q2 = sum dx P2.  Then dL/dmean = (cx P1 + cy P2,
-// cy P1 + cz P2), dL/dconic = (-Q1 / 2, -Q2, -P5 / 2) (converted to dL/dcov2d
-// per (tile, entry), before any sum over tiles), dL/dcolour the sums of
-// alpha T dL/dpixel and dL/dopacity = S0 / opacity.  Value k sits in slot
-// kCol* of the reduction's result.
+// Per (tile, entry) the wave sums nine values over its 128 pixels, from
+// dpw = dL/dpower and aT = alpha T of each: S0 = sum dpw, P1 = sum dpw e,
+// P2 = sum dpw dy, Q1 = sum dpw e^2, Q2 = sum dpw e dy, P5 = sum dpw dy^2 and
+// the colours C = sum aT dL/dpixel, where e = dx + rho dy with the entry's
+// rho = cy / cx (ridge_slope).  The pixel's offset times the conic is then
+//   wx = cx dx + cy dy = cx e + r dy,   r = cy - cx rho,
+//   wy = cy dx + cz dy = cy e + k dy,   k = cz - cy rho,
+// exactly for any rho (r and k are one fused multiply-add each), and the
+// reference's sums (rasterize_backward.cu:163-176, 211-221) are dL/dmean =
+// sum dpw (wx, wy), dL/dcov2d = sum dpw (wx^2 / 2, wx wy, wy^2 / 2) (the
+// conversion from dL/dconic, a congruence), dL/dcolour = C and dL/dopacity =
+// S0 / opacity.  With rho = 0 they are sums about dx and dy, whose second
+// moments a needle-shaped splat's conic cancels to a small remainder (wx^2
+// from cx^2 dx^2, cx cy dx dy and cy^2 dy^2); along the ridge they do not
+// cancel.
+// kGroup entries are walked and summed together, so that the sums' share per
+// entry is a quarter of one reduction:
+// - walking, a lane forms its two pixels' terms of the four entries and leaves
+//   them in LDS, the dpw pairs and then the alpha T pairs;
+// - each is read back transposed, lane 4b + j taking entry j's terms of the
+//   four lanes of quad b (four columns, two rows);
+// - it sums the quad's dpw moments about entry j's mean: about a centre shared by the entries a matrix product could
+//   form them, but where little beyond one pixel beside the mean blends, e^2
+//   would be the difference of numbers thousands of times its size;
+// - the colours' weights dL/dpixel are no entry's own, so their products are
+//   matrix instructions (v_mfma_f32_4x4x1, fp32: sixteen 4x4 outer products,
+//   one per quad, accumulated over the quad's eight pixels);
+// - the sixteen quads are summed (permlane swaps and row rotations).
 constexpr int kTerms = 9;
+constexpr int kGroup = 4;               // entries per matrix-instruction group
+constexpr int kGroupPitch = kWave + 1;  // float2s per entry; +1: transposed reads hit all banks
+constexpr int kS0 = 0, kP1 = 1, kQ1 = 2, kP2 = 3, kQ2 = 4, kP5 = 5, kC0 = 6, kC1 = 7, kC2 = 8;
 
-// dL/dcov2d (a, b, c) from dL/dconic (x, y full off-diagonal, z) for conic =
-// (cx, cy, cz) = cov^-1 (rasterize_backward.cu:211-221).
-__device__ __forceinline__ void conic_to_cov_grad(float cx, float cy, float cz, float dx, float dy,
-                                                  float dz, float out[3]) {
-    const float gx = dx, gy = 0.5f * dy, gz = dz;
-    out[0] = -(cx * cx * gx + 2.0f * cx * cy * gy + cy * cy * gz);
-    out[1] = -2.0f * (cx * cy * gx + (cx * cz + cy * cy) * gy + cy * cz * gz);
-    out[2] = -(cy * cy * gx + 2.0f * cy * cz * gy + cz * cz * gz);
+// Which of the nine sums lane l holds after group_sums, of entry l & 3 (-1:
+// none): by row l >> 4 and quad of the row (l >> 2) & 3.
+__device__ __forceinline__ int group_value_of_lane(int l) {
+    const int row = l >> 4;
+    switch ((l >> 2) & 3) {
+        case 0: return row == 0 ? kS0 : row == 1 ? kP1 : row == 2 ? kC0 : kC1;
+        case 1: return row == 0 ? kQ1 : row == 1 ? kP2 : row == 2 ? kC2 : kP5;
+        case 2: return row == 0 ? kQ2 : -1;
+        default: return -1;
+    }
+}
+
+// The weights of the quad's colour products, element i = l & 3 of lane l:
+// dL/dpixel (r, g, b, 0) of quad lane s's pixel k.
+struct GroupWeights {
+    float g[2][4];
+};
+
+template <int kLane>
+__device__ __forceinline__ float quad_lane(float v) {
+    return dpp_move<kLane * 0x55>(v);  // quad_perm [kLane x 4]
+}
+
+__device__ __forceinline__ GroupWeights group_weights(const BwdPixel (&p)[2]) {
+    const int i = lane_id() & 3;
+    GroupWeights w;
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        auto pick = [&](float r, float g, float b) {
+            return i == 0 ? r : i == 1 ? g : i == 2 ? b : 0.0f;
+        };
+        w.g[k][0] = pick(quad_lane<0>(p[k].g0), quad_lane<0>(p[k].g1), quad_lane<0>(p[k].g2));
+        w.g[k][1] = pick(quad_lane<1>(p[k].g0), quad_lane<1>(p[k].g1), quad_lane<1>(p[k].g2));
+        w.g[k][2] = pick(quad_lane<2>(p[k].g0), quad_lane<2>(p[k].g1), quad_lane<2>(p[k].g2));
+        w.g[k][3] = pick(quad_lane<3>(p[k].g0), quad_lane<3>(p[k].g1), quad_lane<3>(p[k].g2));
+    }
+    return w;
+}
+
+// The nine sums of a group's entries over the wave's pixels; lane l returns
+// sum group_value_of_lane(l) of entry l & 3.  terms: the wave's LDS; x0: the
+// quad's first column, y: its rows; mean, rho: of entry l & 3.  All 64 lanes must
+// be active.
+__device__ __forceinline__ float group_sums(float2* terms, const GroupWeights& wt,
+                                            const BwdTerms (&q)[kGroup][2], float x0,
+                                            const float (&y)[2], const float2& mean, float rho) {
+#pragma clang fp contract(fast)
+    const int l = lane_id();
+    const float2* mine = terms + (l & 3) * kGroupPitch + (l & ~3);
+    // the wave's own stores, read by its other lanes: LDS serves a wave's
+    // accesses in order, and the compiler keeps them so
+    auto order = [] {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    };
+#pragma unroll
+    for (int s = 0; s < kGroup; ++s)
+        terms[s * kGroupPitch + l] = make_float2(q[s][0].dpw, q[s][1].dpw);
+    order();
+    const float dx0 = x0 - mean.x, dy0 = y[0] - mean.y, dy1 = y[1] - mean.y;
+    const float b0 = dx0 + rho * dy0, b1 = dx0 + rho * dy1;
+    float S[2], P[2], Q[2];  // per row: sums of dpw, dpw e, dpw e^2
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+        const float2 t = mine[s];
+        const float e0 = b0 + (float)s, e1 = b1 + (float)s;
+        const float f0 = e0 * t.x, f1 = e1 * t.y;
+        S[0] = s == 0 ? t.x : S[0] + t.x;
+        S[1] = s == 0 ? t.y : S[1] + t.y;
+        P[0] = s == 0 ? f0 : P[0] + f0;
+        P[1] = s == 0 ? f1 : P[1] + f1;
+        Q[0] = s == 0 ? e0 * f0 : Q[0] + e0 * f0;
+        Q[1] = s == 0 ? e1 * f1 : Q[1] + e1 * f1;
+    }
+    order();
+#pragma unroll
+    for (int s = 0; s < kGroup; ++s)
+        terms[s * kGroupPitch + l] = make_float2(q[s][0].aT, q[s][1].aT);
+    order();
+    f32x4 c = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+        const float2 t = mine[s];
+        c = __builtin_amdgcn_mfma_f32_4x4x1f32(wt.g[0][s], t.x, c, 0, 0, 0);
+        c = __builtin_amdgcn_mfma_f32_4x4x1f32(wt.g[1][s], t.y, c, 0, 0, 0);
+    }
+    order();
+    const float S0 = S[0] + S[1], P1 = P[0] + P[1], Q1 = Q[0] + Q[1];
+    const float g0 = dy0 * S[0], g1 = dy1 * S[1];
+    const float P2 = g0 + g1;
+    const float P5 = dy0 * g0 + dy1 * g1;
+    const float Q2 = dy0 * P[0] + dy1 * P[1];
+    // over the quads: lanes 0-31 keep the first of each pair, 32-63 the second
+    const float f0 = fold32(S0, c[0]);
+    const float f1 = fold32(P1, c[1]);
+    const float f2 = fold32(Q1, c[2]);
+    const float f3 = fold32(P2, P5);
+    // Q2 alone: its swaps take a register that is no longer needed (what it
+    // leaves in lanes 32-63 and in rows 1 and 3 is kept by nobody)
+    const float f4 = fold32(Q2, g0);
+    float h0 = fold16(f0, f1);  // rows: S0, P1, C0, C1
+    float h1 = fold16(f2, f3);  // rows: Q1, P2, C2, P5
+    float h2 = fold16(f4, g1);  // row 0: Q2
+    h0 += dpp_move<kDppRowRor8>(h0);
+    h1 += dpp_move<kDppRowRor8>(h1);
+    h2 += dpp_move<kDppRowRor8>(h2);
+    h0 += dpp_move<kDppRowRor4>(h0);
+    h1 += dpp_move<kDppRowRor4>(h1);
+    h2 += dpp_move<kDppRowRor4>(h2);
+    // formed with every lane active: the selects below must not draw the last
+    // adds into branches, away from their lane moves
+    asm volatile("" : "+v"(h0), "+v"(h1), "+v"(h2));
+    const int r = (l >> 2) & 3;
+    return r == 0 ? h0 : r == 1 ? h1 : h2;
+}
+
+// The slope rho of a staged entry's ridge, from the record's a = -cx/2 (A.z) and
+// b = -cy (A.w); 0 where the conic is not positive in x or the slope no number.
+__device__ __forceinline__ float ridge_slope(const float4& A) {
+    const float rho = (0.5f * A.w) / A.z;
+    return (A.z < 0.0f && fabsf(rho) < 1e6f) ? rho : 0.0f;
 }
 
 // Long tiles' backward runs as two work items (tile_order_kernel picks them).
@@ -471,21 +660,145 @@ constexpr int kSplitNum = 37, kSplitDen = 100;
 // Most tiles split per backward launch (the launch has this many extra groups).
 constexpr int kSplitMax = 256;
 
-// The entries of one 64-entry chunk of a staged batch [lo, lo + cnt) that a
-// wave walks, one ballot each: bit e of `walk` for entry c0 + e when it is in
-// the batch, within the wave's largest n_contrib and its strip bit is set;
-// bit e of `fast` for its fast-exp flag.  Lane e reads entry c0 + e's bits.
-struct ChunkMasks {
-    uint64_t walk, fast;
+// The entries of one 64-entry chunk of a staged batch [lo, lo + cnt) that a wave
+// walks: those within its largest n_contrib whose strip bit is set, back to
+// front, as byte offsets of their places in s_a; filled up with the none entry
+// to a whole number of groups.  One ballot and one store per wave: the walk then
+// finds its entries without scalar work.
+struct ChunkList {
+    int count;
+    bool plain;   // all of them are
+    bool within;  // all of them lie within every pixel's n_contrib
 };
-template <int kBatch>
-__device__ __forceinline__ ChunkMasks chunk_masks(const float4* s_c, int c0, int cnt, int lo,
-                                                  int wave_last, uint32_t my_bit) {
-    const int e = c0 + (int)(threadIdx.x & 63);
+template <int kPix, int kBatch>
+__device__ __forceinline__ ChunkList chunk_list(const float2* s_c, int c0, int cnt, int lo,
+                                                int wave_last, uint32_t my_bit,
+                                                const int (&last)[kPix], int* list) {
+    const int l = lane_id();
+    const int e = c0 + l;
     const bool in = e < cnt;
-    const uint32_t b = in ? __float_as_uint(s_c[min(e, kBatch - 1)].w) : 0u;
-    return ChunkMasks{ballot(in && lo + e + 1 <= wave_last && (b & my_bit) != 0u),
-                      ballot((b & kFastExpBit) != 0u)};
+    const uint32_t b = in ? __float_as_uint(s_c[min(e, kBatch - 1)].y) : 0u;
+    const uint64_t walk = ballot(in && lo + e + 1 <= wave_last && (b & my_bit) != 0u);
+    const uint64_t plain = ballot((b & kPlainBit) != 0u);
+    const int end = (min(c0 + kWave, cnt) - 1) * (int)sizeof(float4);
+    bool beyond = false;
+#pragma unroll
+    for (int k = 0; k < kPix; ++k) beyond |= last[k] < end;
+    ChunkList c{popc64(walk), (walk & ~plain) == 0, ballot(beyond) == 0};
+    if ((walk >> l) & 1u) list[popc64(l == 63 ? 0ull : walk >> (l + 1))] = e * (int)sizeof(float4);
+    if (l < kGroup - 1) list[c.count + l] = kBatch * (int)sizeof(float4);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    return c;
+}
+constexpr int kListSize = kWave + kGroup;
+
+template <typename T>
+__device__ __forceinline__ T staged(const void* base, int offset) {
+    return *reinterpret_cast<const T*>(static_cast<const char*>(base) + offset);
+}
+
+// colour . dL/dpixel of the group's entries for the lane's pixels, [pixel][entry]:
+// the entries' colours (lane l reads entry l & 3's, at `own`) by the lanes' own
+// dL/dpixel, as three outer products per pixel (v_mfma_f32_4x4x1; lane l keeps
+// its pixel's column).
+template <int kPix>
+__device__ __forceinline__ void group_colours(int own, const float4* s_b, const float2* s_c,
+                                              const BwdPixel (&p)[kPix], f32x4 (&cg)[kPix]) {
+    const float2 rg = staged<float2>(s_b, own + (int)sizeof(float2));
+    const float b = staged<float>(s_c, own / 2);
+#pragma unroll
+    for (int k = 0; k < kPix; ++k) {
+        f32x4 c = {0.0f, 0.0f, 0.0f, 0.0f};
+        c = __builtin_amdgcn_mfma_f32_4x4x1f32(rg.x, p[k].g0, c, 0, 0, 0);
+        c = __builtin_amdgcn_mfma_f32_4x4x1f32(rg.y, p[k].g1, c, 0, 0, 0);
+        cg[k] = __builtin_amdgcn_mfma_f32_4x4x1f32(b, p[k].g2, c, 0, 0, 0);
+    }
+}
+
+// The wave's decisions for a group's entries, all of them in straight-line code
+// (independent chains, one test for the whole group): the fast evaluation, then
+// the exact one for the whole wave for every entry that is not plain or has a
+// lane near the threshold.  at: the entries' offsets; last: the offset of the
+// last entry of the batch that each pixel blends.
+template <int kPix>
+struct GroupDecision {
+    float ae[kGroup][kPix];
+    uint64_t clamped[kGroup][kPix];
+    bool any, any_clamped;  // some pixel blends an entry, some alpha is clamped
+};
+__device__ __forceinline__ float staged_power(const float4& A, float c, float fx, float fy) {
+    // the forward's power, bit for bit (blend_power)
+    const float dx = fx - A.x, dy = fy - A.y;
+    return __builtin_fmaf(c * dy, dy, __builtin_fmaf(A.w * dx, dy, (A.z * dx) * dx));
+}
+template <int kPix>
+__device__ __forceinline__ void decide_group(GroupDecision<kPix>& d, const int4& at,
+                                             const ChunkList& cl, float fx, const float (&fy)[kPix],
+                                             const int (&last)[kPix], const float4* s_a,
+                                             const float4* s_b, const float2* s_c) {
+    const int off[kGroup] = {at.x, at.y, at.z, at.w};
+    float4 A[kGroup];
+    float2 B[kGroup];
+#pragma unroll
+    for (int s = 0; s < kGroup; ++s) {
+        A[s] = staged<float4>(s_a, off[s]);
+        B[s] = staged<float2>(s_b, off[s]);
+    }
+    uint64_t within[kGroup][kPix];
+#pragma unroll
+    for (int s = 0; s < kGroup; ++s)
+#pragma unroll
+        for (int k = 0; k < kPix; ++k) within[s][k] = ~0ull;
+    if (!cl.within) {
+#pragma unroll
+        for (int s = 0; s < kGroup; ++s)
+#pragma unroll
+            for (int k = 0; k < kPix; ++k) within[s][k] = ballot(off[s] <= last[k]);
+    }
+    uint64_t act = 0, odd[kGroup], odd_any = 0;
+#pragma unroll
+    for (int s = 0; s < kGroup; ++s) {
+        odd[s] = 0;
+#pragma unroll
+        for (int k = 0; k < kPix; ++k) {
+            act |= decide_fast(staged_power(A[s], B[s].x, fx, fy[k]), B[s].y, within[s][k],
+                               d.ae[s][k], odd[s]);
+            d.clamped[s][k] = 0;
+        }
+        odd_any |= odd[s];
+    }
+    uint64_t clamped = 0;
+    if (odd_any != 0 || !cl.plain) {
+#pragma unroll
+        for (int s = 0; s < kGroup; ++s) {
+            const uint32_t bits = (uint32_t)__builtin_amdgcn_readfirstlane(
+                (int)staged<uint32_t>(s_c, off[s] / 2 + (int)sizeof(float)));
+            if (odd[s] == 0 && (bits & kPlainBit) != 0) continue;
+            const float4 a = staged<float4>(s_a, off[s]);
+            const float2 b = staged<float2>(s_b, off[s]);
+#pragma unroll
+            for (int k = 0; k < kPix; ++k) {
+                act |= decide_exact(staged_power(a, b.x, fx, fy[k]), b.y, within[s][k],
+                                    d.ae[s][k], d.clamped[s][k]);
+                clamped |= d.clamped[s][k];
+            }
+        }
+    }
+    // act may hold an entry's fast decision that the exact one took back: the
+    // group is then summed for nothing
+    d.any = act != 0;
+    d.any_clamped = clamped != 0;
+}
+
+// Per pixel the offset of the last entry of the batch at list position lo that
+// it blends (negative: none).
+template <int kPix, int kBatch>
+__device__ __forceinline__ void last_offsets(const BwdPixel (&p)[kPix], int lo,
+                                             int (&last)[kPix]) {
+#pragma unroll
+    for (int k = 0; k < kPix; ++k)
+        last[k] = min(max(p[k].last - lo - 1, -1), kBatch - 1) * (int)sizeof(float4);
 }
 
 // The pixel state's walk over entries [lo0, hi0), back to front: the same
@@ -496,7 +809,7 @@ __device__ __forceinline__ void state_walk(int lo0, int hi0, int n, int tile, in
                                            const float (&fy)[kPix], BwdPixel (&p)[kPix],
                                            const int32_t* __restrict__ ids,
                                            const BlendRec* __restrict__ recs, float4* s_a,
-                                           float4* s_b, float4* s_c) {
+                                           float4* s_b, float2* s_c, int* list) {
     const int tid = threadIdx.x;
     for (int hi = hi0; hi > lo0; hi -= kBatch) {
         const int lo = max(lo0, hi - kBatch);
@@ -504,38 +817,33 @@ __device__ __forceinline__ void state_walk(int lo0, int hi0, int n, int tile, in
         __syncthreads();
         if (tid < cnt)
             stage_entry<kPix>(recs, ids[start + lo + tid], n, tile, tiles_x, s_a, s_b, s_c,
-                              nullptr, nullptr, tid);
+                              nullptr, tid);
         __syncthreads();
+        int last[kPix];
+        last_offsets<kPix, kBatch>(p, lo, last);
         for (int chunk = ((cnt - 1) / kWave) * kWave; chunk >= 0; chunk -= kWave) {
-            const ChunkMasks cm = chunk_masks<kBatch>(s_c, chunk, cnt, lo, wave_last, my_bit);
-            for (uint64_t todo = cm.walk; todo != 0;) {
-                const int jj = 63 - (int)__builtin_clzll(todo);  // back to front
-                todo ^= 1ull << jj;
-                const int j = chunk + jj;
-                const int contributor = lo + j + 1;
-                const float4 A = s_a[j];
-                const float4 B = s_b[j];
-                const float cb = s_c[j].x;
-                const float dx = fx - A.x;
-                const float adxdx = (A.z * dx) * dx;
-                const float bdx = A.w * dx;
-                BwdDecision d[kPix];
+            const ChunkList cl = chunk_list<kPix, kBatch>(s_c, chunk, cnt, lo, wave_last, my_bit,
+                                                          last, list);
+            for (int i = 0; i < cl.count; i += kGroup) {
+                const int4 at = *reinterpret_cast<const int4*>(list + i);
+                GroupDecision<kPix> d;
+                decide_group<kPix>(d, at, cl, fx, fy, last, s_a, s_b, s_c);
+                if (!d.any) continue;  // as the full walk
+                f32x4 cg[kPix];
+                group_colours<kPix>(list[i + (lane_id() & 3)], s_b, s_c, p, cg);
 #pragma unroll
-                for (int k = 0; k < kPix; ++k) {
-                    d[k].dy = fy[k] - A.y;
-                    d[k].power = __builtin_fmaf(B.x * d[k].dy, d[k].dy,
-                                                __builtin_fmaf(bdx, d[k].dy, adxdx));
+                for (int s = 0; s < kGroup; ++s) {
+#pragma unroll
+                    for (int k = 0; k < kPix; ++k) (void)bwd_update(p[k], d.ae[s][k], cg[k][s]);
                 }
-                decide_entry<kPix>(d, B.y, ((cm.fast >> jj) & 1u) != 0u, contributor, p);
-#pragma unroll
-                for (int k = 0; k < kPix; ++k) (void)bwd_update(p[k], d[k], B, cb);
             }
         }
     }
 }
 
 template <int kPix, int kBatch, bool kSplit>
-__global__ __launch_bounds__(Layout<kPix>::kThreads) void blend_bwd_kernel(
+__global__ __launch_bounds__(Layout<kPix>::kThreads)
+__attribute__((amdgpu_waves_per_eu(kBatch == 64 ? 6 : 4))) void blend_bwd_kernel(
     int n, int H, int W, int tiles_x, uint64_t m, const float* __restrict__ grad, GradStrides gst,
     const int2* __restrict__ ranges, const int32_t* __restrict__ ids,
     const BlendRec* __restrict__ recs, const float* __restrict__ finalT,
@@ -544,11 +852,16 @@ __global__ __launch_bounds__(Layout<kPix>::kThreads) void blend_bwd_kernel(
     const uint32_t* __restrict__ order) {
     constexpr int kWaves = Layout<kPix>::kWaves;
     static_assert(kBatch <= Layout<kPix>::kThreads, "one staged entry per thread");
-    __shared__ float4 s_a[kBatch];
-    __shared__ float4 s_b[kBatch];
-    __shared__ float4 s_c[kBatch];
+    // one place more than the batch: the none entry (stage_none)
+    __shared__ float4 s_a[kBatch + 1];
+    __shared__ float4 s_b[kBatch + 1];
+    __shared__ float2 s_c[kBatch + 1];
+    __shared__ float s_rho[kBatch + 1];
     __shared__ int s_id[kBatch];
-    __shared__ float s_part[kWaves][kTerms][kBatch + 1];  // +1: the 9 writers hit 9 banks
+    // +1: the none entry, and a group's writers hit different banks
+    __shared__ float s_part[kWaves][kTerms][kBatch + 1];
+    __shared__ __attribute__((aligned(16))) int s_list[kWaves][kListSize];
+    __shared__ float2 s_terms[kWaves][kGroup * kGroupPitch];
     __shared__ uint32_t s_max[kWaves];
 
     // Work item.  kSplit (a schedule is given): items 2i and 2i + 1 (i < K) are
@@ -577,7 +890,8 @@ __global__ __launch_bounds__(Layout<kPix>::kThreads) void blend_bwd_kernel(
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // scalar: uniform branches
     const uint32_t my_bit = 1u << wave;
-    const Pixels<kPix> pp = pixels_of<kPix>(tile, tiles_x, W, H);
+    static_assert(kPix == 2, "group_sums takes two pixels per lane");
+    const Pixels<kPix> pp = bwd_pixels_of(tile, tiles_x, W, H);
     const int tx = tile % tiles_x, ty = tile / tiles_x;
     const float fx = (float)pp.px;
     float fy[kPix];
@@ -599,7 +913,15 @@ __global__ __launch_bounds__(Layout<kPix>::kThreads) void blend_bwd_kernel(
     for (int w = 0; w < kWaves; ++w) tile_last = max(tile_last, s_max[w]);
     const int maxc = __builtin_amdgcn_readfirstlane(min((int)tile_last, end - start));
     start = __builtin_amdgcn_readfirstlane(start);
-    const int my_value = columns_value_of_lane(lane);
+    const int my_value = group_value_of_lane(lane);
+    const GroupWeights wt = group_weights(p);
+    const float x0 = (float)(tx * kTileSize + (lane & 12));  // the quad's first column
+    int* list = s_list[wave];
+    if (tid == 0) {  // before the first batch's barriers
+        stage_none(s_a, s_b, s_c, kBatch);
+        s_rho[kBatch] = 0.0f;
+    }
+    float2* terms = s_terms[wave];
     // the entries [lo0, hi0) this item walks with gradients; the front part
     // first walks [mid, maxc) for the pixel state only
     int lo0 = 0, hi0 = maxc;
@@ -609,7 +931,7 @@ __global__ __launch_bounds__(Layout<kPix>::kThreads) void blend_bwd_kernel(
         if (part == kPartFront) {
             hi0 = mid;
             state_walk<kPix, kBatch>(mid, maxc, n, tile, tiles_x, start, wave_last, my_bit, fx,
-                                     fy, p, ids, recs, s_a, s_b, s_c);
+                                     fy, p, ids, recs, s_a, s_b, s_c, list);
         }
     }
 
@@ -620,9 +942,15 @@ __global__ __launch_bounds__(Layout<kPix>::kThreads) void blend_bwd_kernel(
         const int lo = max(lo0, hi - kBatch);
         const int cnt = hi - lo;
         const int g = next_id;
+        // the staging's and the flush's addresses are formed again per batch:
+        // kept through the walk they cost it registers, then scratch
+        int tid = (int)threadIdx.x;
+        asm volatile("" : "+v"(tid));
         __syncthreads();
-        if (tid < cnt)
-            stage_entry<kPix>(recs, g, n, tile, tiles_x, s_a, s_b, s_c, nullptr, s_id, tid);
+        if (tid < cnt) {
+            stage_entry<kPix>(recs, g, n, tile, tiles_x, s_a, s_b, s_c, s_id, tid);
+            s_rho[tid] = ridge_slope(s_a[tid]);
+        }
         if (lo > lo0) {
             const int nlo = max(lo0, lo - kBatch);
             if (tid < lo - nlo) next_id = ids[start + nlo + tid];
@@ -633,63 +961,38 @@ __global__ __launch_bounds__(Layout<kPix>::kThreads) void blend_bwd_kernel(
         for (int e = lane; e < cnt; e += kWave)
 #pragma unroll
             for (int k = 0; k < kTerms; ++k) s_part[wave][k][e] = 0.0f;
-        // 64 entries at a time, back to front, the walked ones found with a
-        // scalar find-last over one ballot
+        int last[kPix];
+        last_offsets<kPix, kBatch>(p, lo, last);
         for (int chunk = ((cnt - 1) / kWave) * kWave; chunk >= 0; chunk -= kWave) {
-            const ChunkMasks cm = chunk_masks<kBatch>(s_c, chunk, cnt, lo, wave_last, my_bit);
-            for (uint64_t todo = cm.walk; todo != 0;) {
-                const int jj = 63 - (int)__builtin_clzll(todo);
-                todo ^= 1ull << jj;
-                const int j = chunk + jj;
-                const int contributor = lo + j + 1;
-                float w9;
-                const float4 A = s_a[j];
-                const float4 Cc = s_c[j];  // (b, -cy/2, qthr, strip bits)
-                const float cb = Cc.x;
-                const float4 B = s_b[j];
-                const float dx = fx - A.x;
-                // blend_power's shared column terms: (a dx) dx and b dx
-                const float adxdx = (A.z * dx) * dx;
-                const float bdx = A.w * dx;
-                BwdDecision d[kPix];
+            const ChunkList cl = chunk_list<kPix, kBatch>(s_c, chunk, cnt, lo, wave_last, my_bit,
+                                                          last, list);
+            for (int i = 0; i < cl.count; i += kGroup) {
+                const int4 at = *reinterpret_cast<const int4*>(list + i);
+                const int own = list[i + (lane & 3)];
+                GroupDecision<kPix> d;
+                decide_group<kPix>(d, at, cl, fx, fy, last, s_a, s_b, s_c);
+                // no pixel blends an entry: the state stays and the sums are zero
+                if (!d.any) continue;
+                f32x4 cg[kPix];
+                group_colours<kPix>(own, s_b, s_c, p, cg);
+                BwdTerms q[kGroup][kPix];
 #pragma unroll
-                for (int k = 0; k < kPix; ++k) {
-                    // the forward's power, bit for bit (blend_power)
-                    d[k].dy = fy[k] - A.y;
-                    d[k].power = __builtin_fmaf(B.x * d[k].dy, d[k].dy,
-                                                __builtin_fmaf(bdx, d[k].dy, adxdx));
-                }
-                decide_entry<kPix>(d, B.y, ((cm.fast >> jj) & 1u) != 0u, contributor, p);
-                // per-lane sums over its pixels, started from the first pixel's terms
-                float S0, P2, P5, c0, c1, c2;
-                {
-                    const BwdTerms t = bwd_update(p[0], d[0], B, cb);
-                    const float e = t.dpw * d[0].dy;
-                    S0 = t.dpw;
-                    P2 = e;
-                    P5 = e * d[0].dy;
-                    c0 = t.aT * p[0].g0;
-                    c1 = t.aT * p[0].g1;
-                    c2 = t.aT * p[0].g2;
-                }
+                for (int s = 0; s < kGroup; ++s)
 #pragma unroll
-                for (int k = 1; k < kPix; ++k) {
-                    const BwdTerms t = bwd_update(p[k], d[k], B, cb);
-                    {
-#pragma clang fp contract(fast)
-                        const float e = t.dpw * d[k].dy;
-                        S0 += t.dpw;
-                        P2 += e;
-                        P5 += e * d[k].dy;
-                        c0 += t.aT * p[k].g0;
-                        c1 += t.aT * p[k].g1;
-                        c2 += t.aT * p[k].g2;
-                    }
+                    for (int k = 0; k < kPix; ++k)
+                        q[s][k] = bwd_update(p[k], d.ae[s][k], cg[k][s]);
+                if (d.any_clamped) {
+#pragma unroll
+                    for (int s = 0; s < kGroup; ++s)
+#pragma unroll
+                        for (int k = 0; k < kPix; ++k)
+                            if (__builtin_amdgcn_inverse_ballot_w64(d.clamped[s][k]))
+                                q[s][k].dpw = 0.0f;
                 }
-                // a wave with no blending pixel (2% of the strip-passing
-                // wave-entries on the bench scene) sums zeros
-                w9 = wave_reduce_columns(S0, P2, P5, c0, c1, c2, dx);
-                if (my_value >= 0) s_part[wave][my_value][j] = w9;
+                const float sum =
+                    group_sums(terms, wt, q, x0, fy, staged<float2>(s_a, own),
+                               staged<float>(s_rho, own / 4));
+                if (my_value >= 0) s_part[wave][my_value][own / (int)sizeof(float4)] = sum;
             }
         }
         __syncthreads();
@@ -707,22 +1010,24 @@ __global__ __launch_bounds__(Layout<kPix>::kThreads) void blend_bwd_kernel(
             }
             if (g >= 0 && any) {
                 float t[kTerms];
-                // the record's -cx/2 (A.z), -cy/2 (C.y), -cz/2 (B.x), opacity (B.y)
-                const float ha = s_a[tid].z, hb = s_c[tid].y, hc = s_b[tid].x, o = s_b[tid].y;
-                const float S0 = tot[kColS0], P1 = tot[kColP1], P2 = tot[kColP2];
-                t[0] = -2.0f * (ha * P1 + hb * P2);  // dL/dmean.x = cx P1 + cy P2
-                t[1] = -2.0f * (hb * P1 + hc * P2);  // dL/dmean.y = cy P1 + cz P2
-                // dL/dcov2d from this (tile, entry)'s dL/dconic (x, full
-                // off-diagonal y, z), converted here as the reference converts
-                // each flushed batch (rasterize_backward.cu:211-221): for a
-                // near-singular covariance the conversion's terms cancel, and
-                // they then cancel at one tile's magnitude instead of at the
-                // Gaussian's total over all its tiles
-                conic_to_cov_grad(-2.0f * ha, -2.0f * hb, -2.0f * hc, -0.5f * tot[kColQ1],
-                                  -tot[kColQ2], -0.5f * tot[kColP5], t + 2);
-                t[5] = tot[kColC0];                  // dL/dcolour
-                t[6] = tot[kColC1];
-                t[7] = tot[kColC2];
+                // the record's -cx/2 (A.z), -cy (A.w), -cz/2 (B.x), opacity (B.y)
+                const float cx = -2.0f * s_a[tid].z, cy = -s_a[tid].w, cz = -2.0f * s_b[tid].x;
+                const float o = s_b[tid].y, rho = s_rho[tid];
+                const float r = __builtin_fmaf(-cx, rho, cy), k = __builtin_fmaf(-cy, rho, cz);
+                const float S0 = tot[kS0], P1 = tot[kP1], P2 = tot[kP2];
+                const float Q1 = tot[kQ1], Q2 = tot[kQ2], P5 = tot[kP5];
+                t[0] = cx * P1 + r * P2;  // dL/dmean: sums of dpw wx, dpw wy
+                t[1] = cy * P1 + k * P2;
+                // dL/dcov2d, formed per (tile, entry) as the reference converts
+                // each flushed batch (rasterize_backward.cu:211-221): what
+                // cancels for a near-singular covariance then cancels at one
+                // tile's magnitude instead of at the Gaussian's total
+                t[2] = 0.5f * (cx * (cx * Q1 + 2.0f * r * Q2) + r * r * P5);
+                t[3] = cx * (cy * Q1 + k * Q2) + r * (cy * Q2 + k * P5);
+                t[4] = 0.5f * (cy * (cy * Q1 + 2.0f * k * Q2) + k * k * P5);
+                t[5] = tot[kC0];                  // dL/dcolour
+                t[6] = tot[kC1];
+                t[7] = tot[kC2];
                 // dL/dopacity: every dpw carries a factor opacity (no pixel
                 // blends the entry when the opacity is 0)
                 t[8] = (S0 == 0.0f) ? 0.0f : S0 / o;
@@ -1086,6 +1391,7 @@ bool bwd_split() {
 constexpr int kMaxDevices = 64;
 struct DeviceFacts {
     int cus = 0;
+    unsigned fwd_resident = 0;
     unsigned bwd_resident = 0;
 };
 DeviceFacts device_facts() {
@@ -1093,18 +1399,22 @@ DeviceFacts device_facts() {
     static DeviceFacts table[kMaxDevices];
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices)
-        return DeviceFacts{1, 1};
+        return DeviceFacts{1, 1, 1};
     std::lock_guard<std::mutex> lock(mu);
     DeviceFacts& f = table[dev];
     if (f.cus == 0) {
-        int per_cu = 0, cus = 0;
+        int per_cu = 0, fwd_per_cu = 0, cus = 0;
         if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) !=
                 hipSuccess ||
             hipOccupancyMaxActiveBlocksPerMultiprocessor(
                 &per_cu, reinterpret_cast<const void*>(&blend_bwd_kernel<2, 64, false>),
+                Layout<2>::kThreads, 0) != hipSuccess ||
+            hipOccupancyMaxActiveBlocksPerMultiprocessor(
+                &fwd_per_cu, reinterpret_cast<const void*>(&blend_fwd_kernel<2>),
                 Layout<2>::kThreads, 0) != hipSuccess)
-            return DeviceFacts{1, 1};
+            return DeviceFacts{1, 1, 1};
         f.cus = std::max(1, cus);
+        f.fwd_resident = (unsigned)std::max(1, fwd_per_cu * f.cus);
         f.bwd_resident = (unsigned)std::max(1, per_cu * f.cus);
     }
     return f;
@@ -1112,8 +1422,17 @@ DeviceFacts device_facts() {
 
 int cu_count() { return device_facts().cus; }
 
-// Whether the backward's whole grid of tiles is resident on the device at once.
-bool bwd_grid_fits(unsigned tiles) { return tiles <= device_facts().bwd_resident; }
+// Whether the forward's whole grid of tiles, two pixels per lane, is resident
+// on the device at once.
+bool fwd_grid_fits(unsigned tiles) { return tiles <= device_facts().fwd_resident; }
+
+// Whether the backward's grid of tiles is resident on the device at once, or
+// so nearly (4/3 of what fits: 4096 tiles) that its longest tiles set its
+// length and the 128-entry batch with the split pays: 720p (3600 tiles) 121 us
+// so and 127 with 64-entry batches, 1080p (8160 tiles) 224 and 209.
+bool bwd_grid_fits(unsigned tiles) {
+    return (uint64_t)tiles * 3 <= (uint64_t)device_facts().bwd_resident * 4;
+}
 
 // Lists that average this many entries per tile or more (the screen bands of
 // config c5 average ~350k) are walked like a resident grid's: 128-entry
@@ -1160,12 +1479,12 @@ hipError_t launch_blend_fwd(int n, int H, int W, const int32_t* ranges, const in
     const auto* rc = static_cast<const BlendRec*>(recs);
     // Two pixels per lane share each entry's record reads, column terms and
     // loop, which pays when the total work sets the kernel's length (1080p:
-    // 135.4 -> 129.6 us).  Where the longest tiles set it (a grid resident at
+    // 135.4 -> 129.6 us with a step per entry).  Where the longest tiles set it (a grid resident at
     // once, or lists averaging 32k entries per tile), one pixel per lane in
     // four 16x4 strips culls finer and exits sooner per wave (720p bench frame
     // 0.4615 ms with two pixels per lane against 0.430; c5's blend_fwd 4.86
     // against 4.3 ms per frame).
-    if (bwd_wide(tiles, m))
+    if (fwd_grid_fits(tiles) || bwd_long_lists(tiles, m))
         hipLaunchKernelGGL(blend_fwd_kernel<1>, dim3(tiles), dim3(Layout<1>::kThreads), 0, st,
                            n, H, W, tiles_x, m, r, ids, rc, img, finalT, ncontrib, order);
     else
@@ -1205,15 +1524,15 @@ hipError_t launch_blend_bwd(int n, int H, int W, const float* grad, const GradSt
     if (tiles == 0) return hipSuccess;
     const auto* r = reinterpret_cast<const int2*>(ranges);
     const auto* rc = static_cast<const BlendRec*>(recs);
-    // With a schedule and the whole grid resident at once, or lists long
+    // With a schedule and the grid (nearly) resident at once, or lists long
     // enough that the longest tiles set the kernel's length, up to kSplitMax
     // of the longest run as two items each.  Otherwise the total work does,
     // and the split's extra state-only walk costs more than it saves.
     const bool wide = bwd_wide(tiles, num_pairs);
     const bool split = order && bwd_split() && wide;
-    // The 64-entry batch halves the work-group's LDS (8 KB), so registers, not
-    // LDS, bound the resident waves; it pays when the grid does not fit on the
-    // device at once.  When it would, the 128-entry batch leaves part of the
+    // The 64-entry batch takes 12.5 KB of LDS (13 work-groups per CU, as many
+    // as its registers allow); it pays when the grid does not fit on the device
+    // at once.  When it would, the 128-entry batch (20 KB) leaves part of the
     // grid to be placed as CUs free up, which balances the long tiles better.
     if (!wide)
         hipLaunchKernelGGL((blend_bwd_kernel<2, 64, false>), dim3(tiles),

@@ -150,6 +150,7 @@ constexpr int kDppQuadXor1 = 0xB1;  // quad_perm [1,0,3,2]
 constexpr int kDppQuadXor2 = 0x4E;  // quad_perm [2,3,0,1]
 constexpr int kDppRowShl4 = 0x104;
 constexpr int kDppRowShr4 = 0x114;
+constexpr int kDppRowRor4 = 0x124;  // lane i <- lane (i - 4) & 15 of the row
 constexpr int kDppRowRor8 = 0x128;  // lane i <- lane i ^ 8 within the row
 
 // lane i <- lane i ^ 4 within the row: two bank-masked moves (the first
@@ -174,61 +175,6 @@ __device__ __forceinline__ float fold16(float a, float b) {
     const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false,
                                                     false);
     return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-
-// The backward's nine wave sums from six per-lane sums, for the blend layout
-// where lanes l, l ^ 16, l ^ 32 and l ^ 48 hold the same pixel column (lane &
-// 15, one dx per lane).  A transposed reduction: each level halves the live
-// registers while doubling the lanes summed.  The 32- and 16-lane levels
-// (permlane swaps) run on the six column-free sums only (S0, P2, P5, c0, c1,
-// c2) and leave column totals; then dx S0, dx^2 S0 and dx P2 are formed per
-// column and the 8-, 4-, 2- and 1-lane levels (row_ror, bank-masked row
-// shifts, quad permutes) finish four registers.  ~27 VALU.  Value k's wave
-// total ends in lane kColLane[k] of the result (and in the lanes of its quad).
-// All 64 lanes must be active.
-constexpr int kColS0 = 0, kColP1 = 1, kColQ1 = 2, kColP2 = 3, kColQ2 = 4, kColP5 = 5,
-              kColC0 = 6, kColC1 = 7, kColC2 = 8;
-constexpr int kColLane[9] = {0, 8, 4, 16, 24, 12, 32, 48, 44};
-
-__device__ __forceinline__ float wave_reduce_columns(float s0, float p2, float p5, float c0,
-                                                     float c1, float c2, float dx) {
-    // lanes 0-31 (rows 0, 1) hold S0, P2, P5; lanes 32-63 (rows 2, 3) c0, c1, c2
-    const float r0 = fold32(s0, c0);
-    const float r1 = fold32(p2, c1);
-    const float r2 = fold32(p5, c2);
-    // column totals: a = (S0, P2, c0, c1) in rows 0-3, b = (P5, -, c2, -): b's
-    // swap takes the first swap's spent register as its partner (its rows 1
-    // and 3, summed into b's rows 1 and 3, reach no lane that holds a value)
-    const auto s01 = __builtin_amdgcn_permlane16_swap(__float_as_uint(r0), __float_as_uint(r1),
-                                                      false, false);
-    const float a = __uint_as_float(s01[0]) + __uint_as_float(s01[1]);
-    const auto s2 = __builtin_amdgcn_permlane16_swap(__float_as_uint(r2), s01[0], false, false);
-    const float b = __uint_as_float(s2[0]) + __uint_as_float(s2[1]);
-    const float t1 = dx * a;   // row 0: dx S0, row 1: dx P2
-    const float t2 = dx * t1;  // row 0: dx^2 S0
-    const int l = lane_id();
-    const bool b3 = (l & 8) != 0;
-    const float u0 = (b3 ? t1 : a) + dpp_move<kDppRowRor8>(b3 ? a : t1);
-    const float u1 = (b3 ? b : t2) + dpp_move<kDppRowRor8>(b3 ? t2 : b);
-    const bool b2 = (l & 4) != 0;
-    float w = (b2 ? u1 : u0) + lane_xor4(b2 ? u0 : u1);
-    w = w + dpp_move<kDppQuadXor2>(w);
-    w = w + dpp_move<kDppQuadXor1>(w);
-    // formed here with every lane active, so the last level stays one DPP add
-    // (a caller that only keeps the value in some lanes would otherwise have
-    // the add sunk into its branch and the lane move split from it)
-    asm volatile("" : "+v"(w));
-    return w;
-}
-
-// Which of the nine values lane l holds after wave_reduce_columns (-1: none).
-// Lane l with l & 3 == 0 holds, in row l >> 4, register (l >> 2) & 3 of the
-// last levels: 0 a, 1 t2, 2 t1, 3 b.
-__device__ __forceinline__ int columns_value_of_lane(int l) {
-    if (l & 3) return -1;
-    for (int k = 0; k < 9; ++k)
-        if (kColLane[k] == l) return k;
-    return -1;
 }
 
 __device__ __forceinline__ uint32_t wave_sum_u32(uint32_t v) {
@@ -307,10 +253,11 @@ constexpr uint32_t kSpinLimit = 1u << 22;
 
 // Per-Gaussian blend record (48 B), built once per frame from the
 // rasterize inputs: (mean.x, mean.y, -conic.x/2, -conic.y), (-conic.z/2,
-// opacity, r, g), (b, -conic.y/2, qthr, -).  The conic terms carry the
+// opacity, r, g), (b, -conic.y/2, qthr, plain).  The conic terms carry the
 // power's -1/2 (exact scalings by powers of two), so the blend evaluates
 // power = fma(c dy, dy, fma(b dx, dy, (a dx) dx)) without the final multiply;
-// the conic itself is -2 times them, exactly.
+// the conic itself is -2 times them, exactly.  The last word is kPlainRecord
+// for a plain record (plain_record), else 0.
 // qthr bounds the quadratic form from above for any pixel that can reach
 // alpha >= 1/255 (conservative; negative when the opacity alone rules every
 // pixel out): the blends use it to skip entries for whole pixel regions
@@ -331,6 +278,25 @@ __device__ __forceinline__ float alpha_q_threshold(float o) {
     return (float)(t + 1e-5 * fabs(t) + 1e-4);
 }
 
+// A plain record, which both blends step without the tests that it cannot fail
+// (and with the bound on the power's terms that they add per tile):
+// - opacity in [0, 0.99): alpha = opacity G is never clamped, as G <= 1;
+// - a conic A, C >= 1e-12, B^2 <= (1 - 4e-5) A C: the power's terms sum to at
+//   most -1.9e-5 of (|a| dx^2 + |c| dy^2), forty times the sum of its roundings,
+//   so the computed power is never positive (the mean 0 or at least 1e-10 from
+//   0 per axis, so no product of an offset underflows);
+// - colours in [0, inf): a weight of 0 adds exactly nothing.
+// NaN anywhere makes a record not plain.
+constexpr float kPlainRecord = 1.0f;
+__device__ __forceinline__ bool plain_record(float mx, float my, float A, float B, float C,
+                                             float opacity, float r, float g, float b) {
+    auto away = [](float m) { return m == 0.0f || fabsf(m) >= 1e-10f; };
+    auto colour = [](float c) { return c >= 0.0f && c < __builtin_inff(); };
+    return opacity >= 0.0f && opacity < kAlphaMax && A >= 1e-12f && C >= 1e-12f &&
+           B * B <= 0.99996f * (A * C) && away(mx) && away(my) && colour(r) && colour(g) &&
+           colour(b);
+}
+
 // Conic = cov^-1 with 1/det first (rasterize.cu:224-232), packed with mean,
 // opacity and colour so the blend loads one 48 B record per list entry.
 __device__ __forceinline__ BlendRec blend_record(float mx, float my, float a, float b, float c,
@@ -341,7 +307,8 @@ __device__ __forceinline__ BlendRec blend_record(float mx, float my, float a, fl
     BlendRec rec;
     rec.a = make_float4(mx, my, -0.5f * cx, -cy);
     rec.b = make_float4(-0.5f * cz, opacity, r, g);
-    rec.c = make_float4(bl, -0.5f * cy, alpha_q_threshold(opacity), 0.0f);
+    rec.c = make_float4(bl, -0.5f * cy, alpha_q_threshold(opacity),
+                        plain_record(mx, my, cx, cy, cz, opacity, r, g, bl) ? kPlainRecord : 0.0f);
     return rec;
 }
 
