@@ -10,19 +10,29 @@
 // reflection and crops the 5-pixel margin of the index map, which leaves
 // exactly those windows) and over the 3 channels.  Images are [H, W, 3] fp32.
 //
-// Two kernels, each one pass over HBM with LDS-staged 2D tiles:
-//   ssim_fwd_kernel   per 32x16 tile: the tile and its 5-pixel halo of both
-//                     images into LDS (one coalesced sweep of the interleaved
-//                     channels), a horizontal then a vertical 11-tap pass for
-//                     the five window moments, the SSIM index, and per window
-//                     the three partial derivatives of the index with respect
-//                     to mu_x, E[x^2] and E[xy] (stored for the backward);
+// Two kernels, each one pass over HBM, on tiles of 32x16 pixels with a halo of
+// five, separable with the vertical pass first:
+//   ssim_fwd_kernel   vertical: a thread per interleaved column (3 channels x 42
+//                     columns, so its loads coalesce as the images lie in HBM)
+//                     and half of the rows takes 18 rows of both images straight
+//                     from memory, forms each product x^2, y^2, xy once and the
+//                     five 11-tap sums of 8 rows, and leaves them in LDS;
+//                     horizontal: a thread per four neighbouring windows of a
+//                     channel takes their 14 columns of the sums from LDS, forms
+//                     the moments, the SSIM index, and per window the three
+//                     partial derivatives of the index with respect to mu_x,
+//                     E[x^2] and E[xy] (stored for the backward);
 //                     per-work-group sums of the index and of |gt - img|;
-//   ssim_bwd_kernel   per tile: the derivative maps and their halo into LDS,
-//                     their 11x11 window sums (the window is symmetric, so the
-//                     adjoint of the moments' blur is the same blur), and
+//   ssim_bwd_kernel   the same two passes over the derivative maps (the window is
+//                     symmetric, so the adjoint of the moments' blur is the same
+//                     blur), then
 //                     dL/dimg = g ((1 - lambda)/(3HW) sgn(img - gt)
 //                               - lambda/(3 n_win) [clamp mask] (B1 + 2 x B2 + y B3)).
+// The images are not staged: what is staged per value is five words once, read
+// 17.5 times, where a horizontal pass from staged images took 75 words of LDS
+// per value.  1920x1080, same run, before and after: forward 78 and 60 us,
+// backward 76 and 47 us.  VALU issue bounds both now (234 and 152 instructions
+// per value, 0.68 and 0.55 of the slots), the loads' latency leaves the rest.
 // Only the loss's own arithmetic is fp32-tolerance work: the convolutions use
 // fused multiply-adds.
 #include <hip/hip_runtime.h>
@@ -39,121 +49,146 @@ namespace {
 constexpr int kLossTW = 32, kLossTH = 16;  // output tile (columns x rows)
 constexpr int kWinR = 5;                   // window radius: 11 taps
 constexpr int kWinTaps = 2 * kWinR + 1;
-constexpr int kInW = kLossTW + 2 * kWinR, kInH = kLossTH + 2 * kWinR;  // 42 x 26
-constexpr int kLossThreads = 256;
-constexpr int kRowElems = kInW * 3;                // floats of one halo row
-constexpr int kHaloElems = kInH * kRowElems;       // floats of a tile + halo
-constexpr int kHaloIters = (kHaloElems + kLossThreads - 1) / kLossThreads;
+constexpr int kInCols = 3 * (kLossTW + 2 * kWinR);  // 126 interleaved columns
+constexpr int kRunV = 8;                            // rows a thread sums vertically
+constexpr int kRunVIn = kRunV + kWinTaps - 1;       // from 18
+constexpr int kRunH = 4;                            // windows a thread forms horizontally
+constexpr int kRunHIn = kRunH + kWinTaps - 1;       // from 14 columns of their channel
+constexpr int kRowRuns = 3 * (kLossTW / kRunH);     // 24 per row
+constexpr int kHTasks = kRowRuns * kLossTH;         // 384
+constexpr int kLossThreads = 384;
+constexpr int kFinalThreads = 256;
+constexpr int kPitch = kInCols + 1;                 // odd: the runs' lanes spread over the banks
+static_assert(kHTasks == kLossThreads && kInCols <= 128 && kLossTH / kRunV * 128 <= kLossThreads,
+              "one run of each kind per thread");
+// A byte offset past every row (12 bytes per pixel, rows of at most 2^31 / 33
+// pixels).
+constexpr uint32_t kOutside = 0xffffff00u;
 constexpr float kC1 = 0.01f * 0.01f, kC2 = 0.03f * 0.03f;
 
 struct Window {
     float w[kWinTaps];
 };
 
-// torch.clamp(v, 0, 1): NaN stays NaN.
-__device__ __forceinline__ float clamp01(float v) { return v < 0.0f ? 0.0f : (v > 1.0f ? 1.0f : v); }
+// torch.clamp(v, 0, 1): NaN stays NaN (IEEE 754-2019 maximum and minimum, one
+// instruction each).
+__device__ __forceinline__ float clamp01(float v) {
+    return __builtin_elementwise_minimum(__builtin_elementwise_maximum(v, 0.0f), 1.0f);
+}
 
 // Windows whose support lies inside the image: centres in [5, H - 5) x [5, W - 5).
 __device__ __forceinline__ bool interior(int y, int x, int H, int W) {
     return y >= kWinR && y < H - kWinR && x >= kWinR && x < W - kWinR;
 }
 
-__global__ __launch_bounds__(kLossThreads) void ssim_fwd_kernel(
+// Adds input i's share, w[i - j] v, to the values j of a run it lies in.
+template <int kRun>
+__device__ __forceinline__ void run_add(float (&m)[kRun], const Window& win, int i, float v) {
+#pragma clang fp contract(fast)
+#pragma unroll
+    for (int j = 0; j < kRun; ++j)
+        if (i - j >= 0 && i - j < kWinTaps) m[j] += win.w[i - j] * v;
+}
+
+// The element at byte offset `at` of row y of a plane of interleaved pixels, 0
+// for a row or a column (kOutside) outside the image: the row is a buffer of its
+// own (a scalar descriptor, y is the wave's), so the halo needs no tests and no
+// vector address arithmetic.
+__device__ __forceinline__ float row_load(const float* plane, int y, int H, int W, uint32_t at) {
+    const uint32_t bytes = (y >= 0 && y < H) ? (uint32_t)W * 12u : 0u;
+    const float* row = plane + (ptrdiff_t)y * W * 3;
+    const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(row), 0, (int)bytes,
+                                                        0x00020000);
+    return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rsrc, (int)at, 0, 0));
+}
+
+// A thread's vertical run: two waves (126 of their lanes, one interleaved column
+// each) take the tile's upper eight rows, two the lower.
+struct VerticalRun {
+    int q, r0;     // column of the halo, first row of the tile
+    uint32_t at;   // the column's byte offset in a row
+    bool active;
+};
+__device__ __forceinline__ VerticalRun vertical_run(int x0, int W) {
+    VerticalRun v;
+    const int pair = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 7);
+    v.q = (int)threadIdx.x & 127;
+    v.r0 = pair * kRunV;
+    v.active = pair < kLossTH / kRunV && v.q < kInCols;
+    const int gx = x0 - kWinR + v.q / 3;
+    v.at = (gx >= 0 && gx < W) ? (uint32_t)((x0 - kWinR) * 3 + v.q) * 4u : kOutside;
+    return v;
+}
+
+__global__ __launch_bounds__(kLossThreads)
+__attribute__((amdgpu_waves_per_eu(5))) void ssim_fwd_kernel(
     int H, int W, const float* __restrict__ img, const float* __restrict__ gt, Window win,
     float* __restrict__ gmaps, float2* __restrict__ partial) {
 #pragma clang fp contract(fast)
-    __shared__ float s_x[3][kInH][kInW];
-    __shared__ float s_y[3][kInH][kInW];
-    __shared__ float s_h[5][kInH][kLossTW];
+    __shared__ float s_v[5][kLossTH][kPitch];
     __shared__ float s_red[2][kLossThreads / kWave];
     const int tid = threadIdx.x;
     const int x0 = blockIdx.x * kLossTW, y0 = blockIdx.y * kLossTH;
     const size_t plane = (size_t)H * W * 3;
 
-    // the tile and its halo, channels interleaved as in HBM, every thread's
-    // loads issued together; |gt - img| of the tile's own pixels on the way
-    float l1 = 0.0f;
-    {
-        float xv[kHaloIters], yv[kHaloIters];
+    float l1 = 0.0f;  // |gt - img| of the tile's own pixels
+    const VerticalRun run = vertical_run(x0, W);
+    if (run.active) {
+        const int q = run.q, r0 = run.r0;
+        const bool own = q >= 3 * kWinR && q < kInCols - 3 * kWinR;
+        float xv[kRunVIn], yv[kRunVIn];
 #pragma unroll
-        for (int it = 0; it < kHaloIters; ++it) {
-            const int e = tid + it * kLossThreads;
-            const int r = e / kRowElems, q = e - r * kRowElems;
-            const int gy = y0 - kWinR + r, gx = x0 - kWinR + q / 3;
-            const bool in = e < kHaloElems && gy >= 0 && gy < H && gx >= 0 && gx < W;
-            const size_t idx = (size_t)gy * W * 3 + (size_t)(x0 - kWinR) * 3 + q;
-            xv[it] = in ? img[idx] : 0.0f;
-            yv[it] = in ? gt[idx] : 0.0f;
+        for (int i = 0; i < kRunVIn; ++i) {
+            xv[i] = row_load(img, y0 + r0 - kWinR + i, H, W, run.at);
+            yv[i] = row_load(gt, y0 + r0 - kWinR + i, H, W, run.at);
+        }
+        float m[5][kRunV] = {};
+#pragma unroll
+        for (int i = 0; i < kRunVIn; ++i) {
+            if (own && i >= kWinR && i < kWinR + kRunV) l1 += fabsf(yv[i] - xv[i]);
+            const float x = clamp01(xv[i]), y = clamp01(yv[i]);
+            run_add(m[0], win, i, x);
+            run_add(m[1], win, i, y);
+            run_add(m[2], win, i, x * x);
+            run_add(m[3], win, i, y * y);
+            run_add(m[4], win, i, x * y);
         }
 #pragma unroll
-        for (int it = 0; it < kHaloIters; ++it) {
-            const int e = tid + it * kLossThreads;
-            if (e >= kHaloElems) continue;
-            const int r = e / kRowElems, q = e - r * kRowElems;
-            const int cx = q / 3, ch = q - cx * 3;
-            if (r >= kWinR && r < kWinR + kLossTH && cx >= kWinR && cx < kWinR + kLossTW)
-                l1 += fabsf(yv[it] - xv[it]);
-            s_x[ch][r][cx] = clamp01(xv[it]);
-            s_y[ch][r][cx] = clamp01(yv[it]);
-        }
+        for (int k = 0; k < 5; ++k)
+#pragma unroll
+            for (int j = 0; j < kRunV; ++j) s_v[k][r0 + j][q] = m[k][j];
     }
     __syncthreads();
 
     float ssum = 0.0f;
-    const int vc = tid & (kLossTW - 1), vr = 2 * (tid / kLossTW);  // 2 window rows per thread
-    for (int ch = 0; ch < 3; ++ch) {
-        // horizontal pass: the five moments of 11 columns, for every halo row
-        for (int t = tid; t < kInH * kLossTW; t += kLossThreads) {
-            const int r = t / kLossTW, c = t - r * kLossTW;
-            float mx = 0.0f, my = 0.0f, xx = 0.0f, yy = 0.0f, xy = 0.0f;
+    {
+        const int r = tid / kRowRuns, u = tid - r * kRowRuns, grp = u / 3, ch = u - 3 * grp;
+        const int c = 3 * kRunH * grp + ch;  // the run's first window and input column
+        float m[5][kRunH] = {};
 #pragma unroll
-            for (int k = 0; k < kWinTaps; ++k) {
-                const float xv = s_x[ch][r][c + k], yv = s_y[ch][r][c + k], w = win.w[k];
-                const float wx = w * xv, wy = w * yv;
-                mx += wx;
-                my += wy;
-                xx += wx * xv;
-                yy += wy * yv;
-                xy += wx * yv;
-            }
-            s_h[0][r][c] = mx;
-            s_h[1][r][c] = my;
-            s_h[2][r][c] = xx;
-            s_h[3][r][c] = yy;
-            s_h[4][r][c] = xy;
-        }
-        __syncthreads();
-        // vertical pass: two windows per thread, from 12 rows
-        float m[2][5] = {};
+        for (int i = 0; i < kRunHIn; ++i)
 #pragma unroll
-        for (int k = 0; k < kWinTaps + 1; ++k) {
-            float v[5];
+            for (int k = 0; k < 5; ++k) run_add(m[k], win, i, s_v[k][r][c + 3 * i]);
+        const int gy = y0 + r;
 #pragma unroll
-            for (int i = 0; i < 5; ++i) v[i] = s_h[i][vr + k][vc];
-            if (k < kWinTaps) {
-#pragma unroll
-                for (int i = 0; i < 5; ++i) m[0][i] += win.w[k] * v[i];
-            }
-            if (k >= 1) {
-#pragma unroll
-                for (int i = 0; i < 5; ++i) m[1][i] += win.w[k - 1] * v[i];
-            }
-        }
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const int gy = y0 + vr + j, gx = x0 + vc;
-            if (!interior(gy, gx, H, W)) continue;
-            const float mux = m[j][0], muy = m[j][1];
+        for (int j = 0; j < kRunH; ++j) {
+            const int gx = x0 + kRunH * grp + j;
+            if (gy >= H || gx >= W) continue;
+            const bool window = interior(gy, gx, H, W);
+            const float mux = m[0][j], muy = m[1][j];
             // the variances clamped at 0 (torch.clamp: NaN stays NaN)
-            const float vxx = m[j][2] - mux * mux, vyy = m[j][3] - muy * muy;
+            const float vxx = m[2][j] - mux * mux, vyy = m[3][j] - muy * muy;
             const float sxx = vxx < 0.0f ? 0.0f : vxx, syy = vyy < 0.0f ? 0.0f : vyy;
-            const float sxy = m[j][4] - mux * muy;
+            const float sxy = m[4][j] - mux * muy;
             const float a1 = 2.0f * mux * muy + kC1, a2 = 2.0f * sxy + kC2;
             const float b1 = mux * mux + muy * muy + kC1, b2 = sxx + syy + kC2;
-            const float rb1 = 1.0f / b1, rb2 = 1.0f / b2;
-            const float inv = rb1 * rb2;
+            // one reciprocal for 1 / b1, 1 / b2 and their product (b1 b2 is at
+            // least C1 C2 = 9e-8): the hardware's, corrected once by its residual
+            const float bb = b1 * b2, r0 = __builtin_amdgcn_rcpf(bb);
+            const float inv = r0 + r0 * (1.0f - bb * r0);
+            const float rb1 = b2 * inv, rb2 = b1 * inv;
             const float s = a1 * a2 * inv;
-            ssum += s;
+            ssum += window ? s : 0.0f;
             if (gmaps) {
                 // dS/dA1 = a2 inv, dS/dA2 = a1 inv, dS/dB1 = -S / b1, dS/dB2 = -S / b2;
                 // A1 = 2 mux muy + C1, A2 = 2 (E[xy] - mux muy) + C2,
@@ -163,12 +198,11 @@ __global__ __launch_bounds__(kLossThreads) void ssim_fwd_kernel(
                 const float dBx = (vxx >= 0.0f) ? dB2 : 0.0f;
                 const float g1 = 2.0f * muy * (dA1 - dA2) + 2.0f * mux * (dB1 - dBx);
                 const size_t idx = ((size_t)gy * W + gx) * 3 + ch;
-                gmaps[idx] = g1;              // dS/dmu_x
-                gmaps[plane + idx] = dBx;     // dS/dE[x^2]
-                gmaps[2 * plane + idx] = 2.0f * dA2;  // dS/dE[xy]
+                gmaps[idx] = window ? g1 : 0.0f;              // dS/dmu_x
+                gmaps[plane + idx] = window ? dBx : 0.0f;     // dS/dE[x^2]
+                gmaps[2 * plane + idx] = window ? 2.0f * dA2 : 0.0f;  // dS/dE[xy]
             }
         }
-        __syncthreads();  // s_h is rewritten for the next channel
     }
     const float ws = wave_sum(ssum), wl = wave_sum(l1);
     if ((tid & (kWave - 1)) == 0) {
@@ -188,13 +222,13 @@ __global__ __launch_bounds__(kLossThreads) void ssim_fwd_kernel(
 
 // out[0] = loss, out[1] = SSIM, out[2] = mean |gt - img|, from the work-groups'
 // partial sums (added in double, in work-group order: deterministic).
-__global__ __launch_bounds__(kLossThreads) void loss_finalize_kernel(
+__global__ __launch_bounds__(kFinalThreads) void loss_finalize_kernel(
     int parts, const float2* __restrict__ partial, double n_win, double n_px, float lambda,
     float* __restrict__ out) {
-    __shared__ double s_a[kLossThreads], s_b[kLossThreads];
+    __shared__ double s_a[kFinalThreads], s_b[kFinalThreads];
     const int tid = threadIdx.x;
     double a = 0.0, b = 0.0;
-    for (int i = tid; i < parts; i += kLossThreads) {
+    for (int i = tid; i < parts; i += kFinalThreads) {
         const float2 p = partial[i];
         a += (double)p.x;
         b += (double)p.y;
@@ -202,7 +236,7 @@ __global__ __launch_bounds__(kLossThreads) void loss_finalize_kernel(
     s_a[tid] = a;
     s_b[tid] = b;
     __syncthreads();
-    for (int s = kLossThreads / 2; s > 0; s >>= 1) {
+    for (int s = kFinalThreads / 2; s > 0; s >>= 1) {
         if (tid < s) {
             s_a[tid] += s_a[tid + s];
             s_b[tid] += s_b[tid + s];
@@ -222,87 +256,59 @@ __global__ __launch_bounds__(kLossThreads) void ssim_bwd_kernel(
     const float* __restrict__ gmaps, float c_l1, float c_ssim, const float* __restrict__ grad_loss,
     float* __restrict__ dimg) {
 #pragma clang fp contract(fast)
-    __shared__ float s_g[3][3][kInH][kInW];  // [map][channel][row][column]
-    __shared__ float s_h[3][kInH][kLossTW];
+    __shared__ float s_v[3][kLossTH][kPitch];
     const int tid = threadIdx.x;
     const int x0 = blockIdx.x * kLossTW, y0 = blockIdx.y * kLossTH;
     const size_t plane = (size_t)H * W * 3;
-    // the derivative maps of the windows centred in the tile and its halo;
-    // zero for windows that are not inside the image.  One map at a time,
-    // every thread's loads of it issued together.
-#pragma unroll 1
-    for (int mp = 0; mp < 3; ++mp) {
-        float v[kHaloIters];
+    const float g = grad_loss ? *grad_loss : 1.0f;
+    // the run's own pixels, loaded ahead of the passes
+    const int r = tid / kRowRuns, u = tid - r * kRowRuns, grp = u / 3, ch = u - 3 * grp;
+    const int gy = y0 + r, gx = x0 + kRunH * grp;
+    float xv[kRunH], yv[kRunH];
 #pragma unroll
-        for (int it = 0; it < kHaloIters; ++it) {
-            const int e = tid + it * kLossThreads;
-            const int r = e / kRowElems, q = e - r * kRowElems;
-            const int gy = y0 - kWinR + r, gx = x0 - kWinR + q / 3;
-            const bool in = e < kHaloElems && gy >= 0 && gy < H && gx >= 0 && gx < W &&
-                            interior(gy, gx, H, W);
-            v[it] = in ? gmaps[mp * plane + (size_t)gy * W * 3 + (size_t)(x0 - kWinR) * 3 + q]
-                       : 0.0f;
-        }
+    for (int j = 0; j < kRunH; ++j) {
+        const bool in = gy < H && gx + j < W;
+        const size_t idx = ((size_t)gy * W + gx + j) * 3 + ch;
+        xv[j] = in ? img[idx] : 0.0f;
+        yv[j] = in ? gt[idx] : 0.0f;
+    }
+    // vertical: the derivative maps of the windows centred in the tile and its
+    // halo (the forward stores 0 for windows that are not inside the image)
+    const VerticalRun run = vertical_run(x0, W);
+    if (run.active) {
+        const int q = run.q, r0 = run.r0;
 #pragma unroll
-        for (int it = 0; it < kHaloIters; ++it) {
-            const int e = tid + it * kLossThreads;
-            if (e >= kHaloElems) continue;
-            const int r = e / kRowElems, q = e - r * kRowElems;
-            const int cx = q / 3, ch = q - cx * 3;
-            s_g[mp][ch][r][cx] = v[it];
+        for (int mp = 0; mp < 3; ++mp) {
+            float v[kRunVIn], m[kRunV] = {};
+#pragma unroll
+            for (int i = 0; i < kRunVIn; ++i)
+                v[i] = row_load(gmaps + mp * plane, y0 + r0 - kWinR + i, H, W, run.at);
+#pragma unroll
+            for (int i = 0; i < kRunVIn; ++i) run_add(m, win, i, v[i]);
+#pragma unroll
+            for (int j = 0; j < kRunV; ++j) s_v[mp][r0 + j][q] = m[j];
         }
     }
-    const float g = grad_loss ? *grad_loss : 1.0f;
     __syncthreads();
-    const int vc = tid & (kLossTW - 1), vr = 2 * (tid / kLossTW);
-    for (int ch = 0; ch < 3; ++ch) {
-        for (int t = tid; t < kInH * kLossTW; t += kLossThreads) {
-            const int r = t / kLossTW, c = t - r * kLossTW;
-            float b0 = 0.0f, b1 = 0.0f, b2 = 0.0f;
+    const int c = 3 * kRunH * grp + ch;
+    float m[3][kRunH] = {};
 #pragma unroll
-            for (int k = 0; k < kWinTaps; ++k) {
-                const float w = win.w[k];
-                b0 += w * s_g[0][ch][r][c + k];
-                b1 += w * s_g[1][ch][r][c + k];
-                b2 += w * s_g[2][ch][r][c + k];
-            }
-            s_h[0][r][c] = b0;
-            s_h[1][r][c] = b1;
-            s_h[2][r][c] = b2;
-        }
-        __syncthreads();
-        float m[2][3] = {};
+    for (int i = 0; i < kRunHIn; ++i)
 #pragma unroll
-        for (int k = 0; k < kWinTaps + 1; ++k) {
-            float v[3];
+        for (int k = 0; k < 3; ++k) run_add(m[k], win, i, s_v[k][r][c + 3 * i]);
 #pragma unroll
-            for (int i = 0; i < 3; ++i) v[i] = s_h[i][vr + k][vc];
-            if (k < kWinTaps) {
-#pragma unroll
-                for (int i = 0; i < 3; ++i) m[0][i] += win.w[k] * v[i];
-            }
-            if (k >= 1) {
-#pragma unroll
-                for (int i = 0; i < 3; ++i) m[1][i] += win.w[k - 1] * v[i];
-            }
-        }
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const int gy = y0 + vr + j, gx = x0 + vc;
-            if (gy >= H || gx >= W) continue;
-            const size_t idx = ((size_t)gy * W + gx) * 3 + ch;
-            const float xv = img[idx], yv = gt[idx];
-            const float xc = clamp01(xv), yc = clamp01(yv);
-            // torch's clamp passes the gradient where 0 <= x <= 1
-            const float ds = (xv >= 0.0f && xv <= 1.0f)
-                                 ? m[j][0] + 2.0f * xc * m[j][1] + yc * m[j][2]
-                                 : 0.0f;
-            // d|gt - x|/dx = -sgn(gt - x) (0 at 0, as torch's abs backward)
-            const float u = yv - xv;
-            const float sg = (u > 0.0f) ? -1.0f : ((u < 0.0f) ? 1.0f : (u != u ? u : 0.0f));
-            dimg[idx] = g * (c_l1 * sg - c_ssim * ds);
-        }
-        __syncthreads();
+    for (int j = 0; j < kRunH; ++j) {
+        if (gy >= H || gx + j >= W) continue;
+        const float x = xv[j], y = yv[j];
+        const float xc = clamp01(x), yc = clamp01(y);
+        // torch's clamp passes the gradient where 0 <= x <= 1
+        const float ds = (x >= 0.0f && x <= 1.0f)
+                             ? m[0][j] + 2.0f * xc * m[1][j] + yc * m[2][j]
+                             : 0.0f;
+        // d|gt - x|/dx = -sgn(gt - x) (0 at 0, as torch's abs backward)
+        const float d = y - x;
+        const float sg = (d > 0.0f) ? -1.0f : ((d < 0.0f) ? 1.0f : (d != d ? d : 0.0f));
+        dimg[((size_t)gy * W + gx + j) * 3 + ch] = g * (c_l1 * sg - c_ssim * ds);
     }
 }
 
@@ -336,7 +342,7 @@ hipError_t launch_l1_dssim_fwd(int H, int W, const float* img, const float* gt, 
                        gaussian_window(), gmaps, static_cast<float2*>(partial));
     const double n_win = 3.0 * (double)(H - 2 * kWinR) * (double)(W - 2 * kWinR);
     const double n_px = 3.0 * (double)H * (double)W;
-    hipLaunchKernelGGL(loss_finalize_kernel, dim3(1), dim3(kLossThreads), 0, st,
+    hipLaunchKernelGGL(loss_finalize_kernel, dim3(1), dim3(kFinalThreads), 0, st,
                        (int)(grid.x * grid.y), static_cast<const float2*>(partial), n_win, n_px,
                        lambda, out);
     return hipGetLastError();
