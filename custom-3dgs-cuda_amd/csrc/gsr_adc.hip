@@ -19,7 +19,8 @@
 //   scan:    one work-group: block offsets of the five counts (kept
 //            originals, kept clones, kept split copies, all split sources,
 //            for the noise rows) and their totals;
-//   gather:  each source writes its kept copies at their final positions:
+//   gather:  each block of 256 sources writes its kept copies at their final
+//            positions, one contiguous run of rows per kind:
 //            [kept originals] [kept clones] [kept first split copies]
 //            [kept second split copies], the reference's order.  Split copies
 //            get mu + R(q) (z * exp(s)) with z the caller's N(0, 1) rows (the
@@ -40,12 +41,15 @@ namespace gsr {
 namespace {
 
 constexpr int kAdcThreads = 256;
-// Elements per thread whose loads copy_rows issues together.
-constexpr int kAdcUnroll = 4;
+// Elements per thread whose loads copy_list issues together.
+constexpr int kAdcUnroll = 8;
 
 // flag bits of a source Gaussian
 constexpr uint8_t kKeepOrig = 1, kKeepClone = 2, kKeepSplit = 4, kSplitSrc = 8, kCloneSrc = 16;
 constexpr int kKinds = 5;
+// Parts of the arrays that the gather's work-groups share out: the wide parameter
+// and its two moments, the other parameters, their first and second moments.
+constexpr int kGatherParts = 6;
 
 __device__ __forceinline__ bool isnan_f(float x) { return x != x; }
 
@@ -146,7 +150,7 @@ __global__ __launch_bounds__(kAdcThreads) void adc_plan_kernel(
 // Exclusive scan of the blocks' counts, per kind, in place; totals[kKinds].
 __global__ __launch_bounds__(1024) void adc_scan_kernel(int blocks, uint32_t* __restrict__ counts,
                                                        uint64_t* __restrict__ totals) {
-    __shared__ uint32_t s_part[kKinds][1024];
+    __shared__ uint32_t s_wave[kKinds][1024 / kWave];
     const int tid = threadIdx.x;
     // each thread a contiguous run of blocks
     const int per = (blocks + 1023) / 1024;
@@ -154,20 +158,27 @@ __global__ __launch_bounds__(1024) void adc_scan_kernel(int blocks, uint32_t* __
     uint32_t sum[kKinds] = {0, 0, 0, 0, 0};
     for (int b = b0; b < b1; ++b)
         for (int k = 0; k < kKinds; ++k) sum[k] += counts[kKinds * (size_t)b + k];
-    for (int k = 0; k < kKinds; ++k) s_part[k][tid] = sum[k];
-    __syncthreads();
-    if (tid < kKinds) {
-        uint32_t run = 0;
-        for (int j = 0; j < 1024; ++j) {
-            const uint32_t v = s_part[tid][j];
-            s_part[tid][j] = run;
-            run += v;
-        }
-        totals[tid] = run;
+    // over the threads: within each wave, then over the sixteen waves' totals
+    const int lane = tid & (kWave - 1), w = tid / kWave;
+    uint32_t incl[kKinds];
+#pragma unroll
+    for (int k = 0; k < kKinds; ++k) {
+        incl[k] = wave_inclusive_scan(sum[k]);
+        if (lane == kWave - 1) s_wave[k][w] = incl[k];
     }
     __syncthreads();
     uint32_t run[kKinds];
-    for (int k = 0; k < kKinds; ++k) run[k] = s_part[k][tid];
+#pragma unroll
+    for (int k = 0; k < kKinds; ++k) {
+        uint32_t before = 0, total = 0;
+#pragma unroll
+        for (int v = 0; v < 1024 / kWave; ++v) {
+            before += v < w ? s_wave[k][v] : 0u;
+            total += s_wave[k][v];
+        }
+        run[k] = before + incl[k] - sum[k];
+        if (tid == 0) totals[k] = total;
+    }
     for (int b = b0; b < b1; ++b)
         for (int k = 0; k < kKinds; ++k) {
             const uint32_t v = counts[kKinds * (size_t)b + k];
@@ -176,53 +187,78 @@ __global__ __launch_bounds__(1024) void adc_scan_kernel(int blocks, uint32_t* __
         }
 }
 
-// Destinations of a block's Gaussians in the new cloud (row indices, or
-// kNoRow): itself, its clone, its two split copies.
-constexpr uint32_t kNoRow = 0xffffffffu;
+// The block's kept sources of one kind (places in the block, in order) and the
+// first of the contiguous rows that they take in the new cloud.
+struct KeptRows {
+    const uint8_t* list;
+    int count;
+    uint64_t row0;
+};
 
-// Copies one [N, W] array of the block's Gaussians to their destinations,
-// element-parallel: the block's source rows are contiguous, so the loads are
-// coalesced, and each destination kind's rows are contiguous too (the order
-// is kept), so are the stores up to the dropped rows.  mode 0: a parameter
-// (every destination gets the value; with `skip_split` the split copies are
-// left to the caller; with `clamp` the value is min(v, clamp_hi), NaN kept);
-// mode 1: a moment (the Gaussian's own row gets the value, new rows zero;
-// `zero_all` zeroes every row).
+// Copies the listed rows of a block's [cnt, W] source rows to consecutive rows
+// of dst, element-parallel over the destination: whole-line stores, loads
+// coalesced up to the dropped rows (cached: the rows left out share their lines,
+// and streaming stores of the short runs cost 30% more).  With `clamp` the value is
+// min(v, hi), NaN kept.  What bounds the pass is HBM (every parameter and moment
+// in once and out once: 1M sources with 12% new rows 311 us, 4.8 TB/s); with one
+// loop over the source elements and four destination lookups each it was VALU
+// issue and one chain of 18 arrays per work-group (519 us).
 template <int W>
-__device__ __forceinline__ void copy_rows(const float* __restrict__ src, float* __restrict__ dst,
-                                          int g0, int cnt, const uint32_t (*s_dst)[kAdcThreads],
-                                          int mode, bool skip_split, bool clamp, float clamp_hi,
-                                          bool zero_all) {
-    const float* sp = src ? src + (size_t)g0 * W : nullptr;
-    const int total = cnt * W;
-    // kAdcUnroll elements per thread and step, their loads issued together
-    for (int e0 = threadIdx.x; e0 < total; e0 += kAdcUnroll * kAdcThreads) {
+__device__ __forceinline__ void copy_list(const float* __restrict__ src, float* __restrict__ dst,
+                                          const KeptRows& k, bool clamp = false,
+                                          float hi = 0.0f) {
+    float* out = dst + (size_t)k.row0 * W;
+    const int total = k.count * W;
+    for (int e0 = (int)threadIdx.x; e0 < total; e0 += kAdcUnroll * kAdcThreads) {
         float v[kAdcUnroll];
 #pragma unroll
         for (int u = 0; u < kAdcUnroll; ++u) {
             const int e = e0 + u * kAdcThreads;
-            v[u] = (sp && e < total) ? sp[e] : 0.0f;
+            const int j = e / W;
+            v[u] = (e < total) ? src[(int)k.list[j] * W + (e - j * W)]
+                               : 0.0f;
         }
 #pragma unroll
         for (int u = 0; u < kAdcUnroll; ++u) {
             const int e = e0 + u * kAdcThreads;
             if (e >= total) break;
-            const int g = e / W, k = e - g * W;
-#pragma unroll
-            for (int d = 0; d < 4; ++d) {
-                const uint32_t row = s_dst[d][g];
-                if (row == kNoRow) continue;
-                if (mode == 0) {
-                    if (skip_split && d >= 2) continue;
-                    float x = v[u];
-                    if (clamp) x = isnan_f(x) ? x : fminf(x, clamp_hi);
-                    dst[(size_t)row * W + k] = x;
-                } else {
-                    dst[(size_t)row * W + k] = (d == 0 && !zero_all) ? v[u] : 0.0f;
-                }
-            }
+            float x = v[u];
+            if (clamp) x = isnan_f(x) ? x : fminf(x, hi);
+            out[e] = x;
         }
     }
+}
+
+template <int W>
+__device__ __forceinline__ void zero_rows(float* __restrict__ dst, const KeptRows& k) {
+    float* out = dst + (size_t)k.row0 * W;
+    for (int e = (int)threadIdx.x; e < k.count * W; e += kAdcThreads)
+        out[e] = 0.0f;
+}
+
+// A parameter's rows: every kept copy gets its source's value (the split copies'
+// mu and s are left to the caller).
+template <int W>
+__device__ __forceinline__ void copy_param(const float* __restrict__ src, float* __restrict__ dst,
+                                           int g0, const KeptRows (&k)[4], bool skip_split,
+                                           bool clamp = false, float hi = 0.0f) {
+    const float* s = src + (size_t)g0 * W;
+    copy_list<W>(s, dst, k[0], clamp, hi);
+    copy_list<W>(s, dst, k[1], clamp, hi);
+    if (skip_split) return;
+    copy_list<W>(s, dst, k[2], clamp, hi);
+    copy_list<W>(s, dst, k[3], clamp, hi);
+}
+
+// A moment's rows: a Gaussian's own row gets the value (zero without a source
+// or with `zero_all`), new rows zero.
+template <int W>
+__device__ __forceinline__ void copy_moment(const float* __restrict__ src, float* __restrict__ dst,
+                                            int g0, const KeptRows (&k)[4], bool zero_all) {
+    if (!dst) return;
+    if (src && !zero_all) copy_list<W>(src + (size_t)g0 * W, dst, k[0]);
+    else zero_rows<W>(dst, k[0]);
+    for (int d = 1; d < 4; ++d) zero_rows<W>(dst, k[d]);
 }
 
 __global__ __launch_bounds__(kAdcThreads) void adc_gather_kernel(
@@ -230,9 +266,8 @@ __global__ __launch_bounds__(kAdcThreads) void adc_gather_kernel(
     const uint32_t* __restrict__ offs, const uint64_t* __restrict__ totals,
     const float* __restrict__ noise, AdcConfig c, AdcCloud out, AdcMoments mout) {
     __shared__ uint32_t s_w[4][kAdcThreads / kWave];
-    __shared__ uint32_t s_dst[4][kAdcThreads];
+    __shared__ uint8_t s_list[3][kAdcThreads];
     const int g0 = blockIdx.x * kAdcThreads;
-    const int cnt = min(kAdcThreads, n - g0);
     const int i = g0 + threadIdx.x;
     const uint8_t f = (i < n) ? flags[i] : 0;
     const int w = threadIdx.x / kWave;
@@ -244,38 +279,54 @@ __global__ __launch_bounds__(kAdcThreads) void adc_gather_kernel(
         if ((threadIdx.x & (kWave - 1)) == 0) s_w[k][w] = (uint32_t)popc64(b);
     }
     __syncthreads();
+    uint32_t held[4], first[4];
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-        uint32_t pre = offs[kKinds * (size_t)blockIdx.x + k];
-        for (int j = 0; j < w; ++j) pre += s_w[k][j];
-        rank[k] += pre;
+        uint32_t pre = 0, all = 0;
+        for (int j = 0; j < kAdcThreads / kWave; ++j) {
+            pre += j < w ? s_w[k][j] : 0u;
+            all += s_w[k][j];
+        }
+        rank[k] += pre;  // within the block
+        held[k] = all;
+        first[k] = offs[kKinds * (size_t)blockIdx.x + k];
     }
+    if (f & kKeepOrig) s_list[0][rank[0]] = (uint8_t)threadIdx.x;
+    if (f & kKeepClone) s_list[1][rank[1]] = (uint8_t)threadIdx.x;
+    if (f & kKeepSplit) s_list[2][rank[2]] = (uint8_t)threadIdx.x;
+    __syncthreads();
     const uint64_t n_orig = totals[0], n_clone = totals[1], n_split = totals[2];
     const uint64_t n_src = totals[3];
-    s_dst[0][threadIdx.x] = (f & kKeepOrig) ? (uint32_t)rank[0] : kNoRow;
-    s_dst[1][threadIdx.x] = (f & kKeepClone) ? (uint32_t)(n_orig + rank[1]) : kNoRow;
-    s_dst[2][threadIdx.x] = (f & kKeepSplit) ? (uint32_t)(n_orig + n_clone + rank[2]) : kNoRow;
-    s_dst[3][threadIdx.x] =
-        (f & kKeepSplit) ? (uint32_t)(n_orig + n_clone + n_split + rank[2]) : kNoRow;
-    __syncthreads();
-    if (cnt <= 0) return;
+    const KeptRows k[4] = {
+        {s_list[0], (int)held[0], first[0]},
+        {s_list[1], (int)held[1], n_orig + first[1]},
+        {s_list[2], (int)held[2], n_orig + n_clone + first[2]},
+        {s_list[2], (int)held[2], n_orig + n_clone + n_split + first[2]}};
     const bool reset = c.reset_opacity != 0;
-    // the parameters (the split copies' mu and s below), then the moments
-    copy_rows<3>(in.p[0], out.p[0], g0, cnt, s_dst, 0, true, false, 0.0f, false);
-    copy_rows<4>(in.p[1], out.p[1], g0, cnt, s_dst, 0, false, false, 0.0f, false);
-    copy_rows<3>(in.p[2], out.p[2], g0, cnt, s_dst, 0, true, false, 0.0f, false);
-    copy_rows<1>(in.p[3], out.p[3], g0, cnt, s_dst, 0, false, reset, c.reset_logit, false);
-    copy_rows<3>(in.p[4], out.p[4], g0, cnt, s_dst, 0, false, false, 0.0f, false);
-    copy_rows<45>(in.p[5], out.p[5], g0, cnt, s_dst, 0, false, false, 0.0f, false);
-    for (int m = 0; m < 2; ++m) {
-        const int o = 6 * m;
-        if (mout.p[o + 0]) copy_rows<3>(min_.p[o + 0], mout.p[o + 0], g0, cnt, s_dst, 1, false, false, 0.0f, false);
-        if (mout.p[o + 1]) copy_rows<4>(min_.p[o + 1], mout.p[o + 1], g0, cnt, s_dst, 1, false, false, 0.0f, false);
-        if (mout.p[o + 2]) copy_rows<3>(min_.p[o + 2], mout.p[o + 2], g0, cnt, s_dst, 1, false, false, 0.0f, false);
-        if (mout.p[o + 3]) copy_rows<1>(min_.p[o + 3], mout.p[o + 3], g0, cnt, s_dst, 1, false, false, 0.0f, reset);
-        if (mout.p[o + 4]) copy_rows<3>(min_.p[o + 4], mout.p[o + 4], g0, cnt, s_dst, 1, false, false, 0.0f, false);
-        if (mout.p[o + 5]) copy_rows<45>(min_.p[o + 5], mout.p[o + 5], g0, cnt, s_dst, 1, false, false, 0.0f, false);
+    // one part of the arrays per work-group (blockIdx.y), so that a block's
+    // copies wait on each other's loads in six places and not in one chain
+    const int part = (int)blockIdx.y;
+    if (part < 3) {
+        const int o = 6 * (part - 1);
+        if (part == 0) copy_param<45>(in.p[5], out.p[5], g0, k, false);
+        else copy_moment<45>(min_.p[o + 5], mout.p[o + 5], g0, k, false);
+        return;
     }
+    if (part > 3) {
+        const int o = 6 * (part - 4);
+        copy_moment<3>(min_.p[o + 0], mout.p[o + 0], g0, k, false);
+        copy_moment<4>(min_.p[o + 1], mout.p[o + 1], g0, k, false);
+        copy_moment<3>(min_.p[o + 2], mout.p[o + 2], g0, k, false);
+        copy_moment<1>(min_.p[o + 3], mout.p[o + 3], g0, k, reset);
+        copy_moment<3>(min_.p[o + 4], mout.p[o + 4], g0, k, false);
+        return;
+    }
+    // the parameters (the split copies' mu and s below)
+    copy_param<3>(in.p[0], out.p[0], g0, k, true);
+    copy_param<4>(in.p[1], out.p[1], g0, k, false);
+    copy_param<3>(in.p[2], out.p[2], g0, k, true);
+    copy_param<1>(in.p[3], out.p[3], g0, k, false, reset, c.reset_logit);
+    copy_param<3>(in.p[4], out.p[4], g0, k, false);
     if (i >= n) return;
     // the kept original's and clone's mu and s were copied above; the split
     // copies' are the perturbed ones
@@ -297,9 +348,9 @@ __global__ __launch_bounds__(kAdcThreads) void adc_gather_kernel(
              1.0f - 2.0f * (qx * qx + qy * qy)}};
         const float sc[3] = {exp_gs(sv[0]), exp_gs(sv[1]), exp_gs(sv[2])};
         for (int copy = 0; copy < 2; ++copy) {
-            const size_t d = (size_t)s_dst[2 + copy][threadIdx.x];
+            const size_t d = (size_t)(k[2 + copy].row0 + rank[2]);
             // the split source's noise row: copy k of source j is row k n_src + j
-            const float* z = noise + 3 * ((size_t)copy * n_src + rank[3]);
+            const float* z = noise + 3 * ((size_t)copy * n_src + first[3] + rank[3]);
             float smp[3];
             for (int a = 0; a < 3; ++a) smp[a] = z[a] * sc[a];
             float* om = out.p[0] + 3 * d;
@@ -354,7 +405,7 @@ hipError_t launch_adc_gather(int n, const AdcCloud& in, const AdcMoments& min_,
     const uint8_t* flags = reinterpret_cast<const uint8_t*>(base + 256);
     const uint32_t* offs =
         reinterpret_cast<const uint32_t*>(base + 256 + ((size_t)n + 255) / 256 * 256);
-    hipLaunchKernelGGL(adc_gather_kernel, dim3(blocks), dim3(kAdcThreads), 0, st, n, in, min_,
+    hipLaunchKernelGGL(adc_gather_kernel, dim3(blocks, kGatherParts), dim3(kAdcThreads), 0, st, n, in, min_,
                        flags, offs, totals_dev, noise, c, out, mout);
     return hipGetLastError();
 }
