@@ -55,9 +55,10 @@ __device__ __forceinline__ uint32_t uniform(uint32_t v) {
 // i % 8); renumbered, the XCD of work-group i takes a contiguous share of the
 // indices, so neighbouring segments (whose runs of a tile share cache lines)
 // are written through the same L2, which merges them into whole lines.
-// Grids that are not a multiple of 8 keep their order.
-__device__ __forceinline__ uint32_t xcd_group() {
-    const uint32_t g = blockIdx.x, n = gridDim.x;
+// Grids (or parts of n work-groups of one) that are not a multiple of 8 keep
+// their order.
+__device__ __forceinline__ uint32_t xcd_group(uint32_t n) {
+    const uint32_t g = blockIdx.x;
     return (n % 8u == 0u) ? (g % 8u) * (n / 8u) + g / 8u : g;
 }
 
@@ -112,28 +113,30 @@ __device__ __forceinline__ uint16_t local_rect(const Rect& t, int ox, int oy) {
     return (uint16_t)(lx0 | ((lx1 - lx0 - 1) << 3) | (ly0 << 6) | ((ly1 - ly0 - 1) << 9));
 }
 
+__device__ __forceinline__ RankLane rect_lane(uint32_t g, uint2 packed) {
+    RankLane L{0u, 0, 0, 0u, 0u, false, Rect{0, 0, 0, 0}};
+    const Rect t = unpack_rect(packed);
+    if (t.x1 > t.x0 && t.y1 > t.y0) {
+        L.g = g;
+        L.t = t;
+        L.bx0 = t.x0 >> 3;
+        L.by0 = t.y0 >> 3;
+        L.bw = (uint32_t)(((t.x1 + 7) >> 3) - L.bx0);
+        L.bh = (uint32_t)(((t.y1 + 7) >> 3) - L.by0);
+        L.has = true;
+    }
+    return L;
+}
+
 // drects: the rectangles already in depth order (rank_rects_kernel), read in
 // rank order instead of by Gaussian id.
 __device__ __forceinline__ RankLane rank_lane(int n, const uint32_t* __restrict__ perm,
                                               const uint2* __restrict__ rects,
                                               const uint2* __restrict__ drects, int64_t r) {
-    RankLane L{0u, 0, 0, 0u, 0u, false, Rect{0, 0, 0, 0}};
-    if (r < n) {
-        const uint32_t g = perm[r];
-        if (g < (uint32_t)n) {
-            const Rect t = unpack_rect(drects ? drects[r] : rects[g]);
-            if (t.x1 > t.x0 && t.y1 > t.y0) {
-                L.g = g;
-                L.t = t;
-                L.bx0 = t.x0 >> 3;
-                L.by0 = t.y0 >> 3;
-                L.bw = (uint32_t)(((t.x1 + 7) >> 3) - L.bx0);
-                L.bh = (uint32_t)(((t.y1 + 7) >> 3) - L.by0);
-                L.has = true;
-            }
-        }
-    }
-    return L;
+    const uint32_t g = (r < n) ? perm[r] : 0xffffffffu;
+    uint2 packed = make_uint2(0u, 0u);
+    if (g < (uint32_t)n) packed = drects ? drects[r] : rects[g];
+    return rect_lane(g, packed);
 }
 
 // Level-1 work item of one wave: chunk c of 64 depth ranks against window w
@@ -212,19 +215,21 @@ struct RecordArgs {
     uint32_t first;
 };
 
+__device__ __forceinline__ void write_record(int n, int i, const RecordArgs& ra) {
+    if (!ra.recs || i >= n) return;
+    const float mx = ra.mean2d[2 * (size_t)i], my = ra.mean2d[2 * (size_t)i + 1];
+    const float a = ra.cov2d[3 * (size_t)i], b = ra.cov2d[3 * (size_t)i + 1],
+                c = ra.cov2d[3 * (size_t)i + 2];
+    ra.recs[i] = blend_record(mx, my, a, b, c, ra.alpha[i], ra.colors[3 * (size_t)i],
+                              ra.colors[3 * (size_t)i + 1], ra.colors[3 * (size_t)i + 2]);
+}
+
 __global__ __launch_bounds__(kThreads) void block_count_kernel(
     int n, const uint32_t* __restrict__ perm, const uint2* __restrict__ rects,
     const uint2* __restrict__ drects, BlockGrid bg,
     int chunks, int windows, int cstride, uint32_t* __restrict__ counts, RecordArgs ra) {
-    if (ra.recs && blockIdx.x >= ra.first) {
-        const int i = (int)(blockIdx.x - ra.first) * kThreads + (int)threadIdx.x;
-        if (i < n) {
-            const float mx = ra.mean2d[2 * (size_t)i], my = ra.mean2d[2 * (size_t)i + 1];
-            const float a = ra.cov2d[3 * (size_t)i], b = ra.cov2d[3 * (size_t)i + 1],
-                        c = ra.cov2d[3 * (size_t)i + 2];
-            ra.recs[i] = blend_record(mx, my, a, b, c, ra.alpha[i], ra.colors[3 * (size_t)i],
-                                      ra.colors[3 * (size_t)i + 1], ra.colors[3 * (size_t)i + 2]);
-        }
+    if (blockIdx.x >= ra.first) {
+        write_record(n, (int)(blockIdx.x - ra.first) * kThreads + (int)threadIdx.x, ra);
         return;
     }
     const int lane = lane_id();
@@ -309,6 +314,127 @@ __global__ __launch_bounds__(kThreads) void block_scatter_kernel(
                 lists[p] = L.g;
                 lrects[p] = local_rect(L.t, sx * 8, sy * 8);
             }
+        }
+    }
+}
+
+// Level 1 at large counts: one work-group takes 512 consecutive ranks against
+// all blocks.  The kernels above form a chunk's masks again for each window of 64
+// blocks, and keep a count per block and chunk of 64: 160 MB of scattered words
+// at 5M Gaussians on a 4K screen (510 blocks).  Here a chunk's masks are formed
+// once and kept in LDS, a count covers the work-group's 8 chunks, and a block's
+// entries of a work-group (5 at that size) are written together.  With the
+// rectangles' gather in the count, counts, scan and scatter of that frame take
+// 522 us (the kernels above 1183), of a million Gaussians at 1080p 66 (106).
+// The scatter (330 us there) is bound by its stores, one L2 request per entry
+// and array.  1024 ranks per work-group: 562; 256: 561.
+// Screens of at most 64 x 64 blocks: lane j holds block row j and column j.
+constexpr int kGroupThreads = 512;
+constexpr int kGroupChunks = kGroupThreads / kWave;
+
+struct GroupMasks {
+    uint64_t row[kGroupChunks][kWave];  // chunk's lanes meeting block row j
+    uint64_t col[kGroupChunks][kWave];  // chunk's lanes meeting block column j
+};
+
+__device__ __forceinline__ void group_masks(const RankLane& L, const BlockGrid& bg,
+                                            uint64_t* __restrict__ row,
+                                            uint64_t* __restrict__ col) {
+    const int lane = lane_id();
+    const uint64_t lanes = ballot(L.has);
+    uint64_t rowv = 0, colv = 0;
+    for (int j = 0; j < bg.bh; ++j) {
+        const uint64_t m = lanes & ballot((uint32_t)(j - L.by0) < L.bh);
+        rowv = (lane == j) ? m : rowv;
+    }
+    for (int j = 0; j < bg.bw; ++j) {
+        const uint64_t m = ballot((uint32_t)(j - L.bx0) < L.bw);
+        colv = (lane == j) ? m : colv;
+    }
+    row[lane] = rowv;
+    col[lane] = colv;
+}
+
+// counts[b * gstride + group] = how many of the group's ranks meet block b, and
+// drects[r] = rects[perm[r]].  The records as in block_count_kernel.
+__global__ __launch_bounds__(kGroupThreads) void group_count_kernel(
+    int n, const uint32_t* __restrict__ perm, const uint2* __restrict__ rects,
+    uint2* __restrict__ drects, BlockGrid bg, int groups, int gstride,
+    uint32_t* __restrict__ counts, RecordArgs ra) {
+    __shared__ GroupMasks s;
+    const int tid = threadIdx.x, wave = tid >> 6;
+    if (blockIdx.x >= ra.first) {
+        write_record(n, (int)(blockIdx.x - ra.first) * kGroupThreads + tid, ra);
+        return;
+    }
+    const int group = (int)xcd_group(ra.first);
+    if (group >= groups) return;
+    const int64_t r = (int64_t)group * kGroupThreads + tid;
+    const uint32_t g = (r < n) ? perm[r] : 0xffffffffu;
+    const uint2 rc = (g < (uint32_t)n) ? rects[g] : make_uint2(0u, 0u);
+    if (r < n) drects[r] = rc;
+    group_masks(rect_lane(g, rc), bg, s.row[wave], s.col[wave]);
+    __syncthreads();
+    for (int b = tid; b < bg.nb; b += kGroupThreads) {
+        const int sy = b / bg.bw, sx = b - sy * bg.bw;
+        uint32_t c = 0;
+#pragma unroll
+        for (int j = 0; j < kGroupChunks; ++j) c += (uint32_t)popc64(s.row[j][sy] & s.col[j][sx]);
+        counts[(size_t)b * gstride + group] = c;
+    }
+}
+
+// As block_scatter_kernel, from the groups' positions and the rectangles in
+// depth order; blocks are taken 512 at a time.
+__global__ __launch_bounds__(kGroupThreads) void group_scatter_kernel(
+    int n, const uint32_t* __restrict__ perm, const uint2* __restrict__ drects, BlockGrid bg,
+    int groups, int gstride, const uint32_t* __restrict__ pos, uint32_t* __restrict__ lists,
+    uint16_t* __restrict__ lrects, uint64_t cap) {
+    __shared__ GroupMasks s;
+    // per block of the window: the group's position, and what the chunks before
+    // a chunk add to it
+    __shared__ uint32_t s_start[kGroupThreads];
+    __shared__ uint16_t s_rel[kGroupChunks][kGroupThreads];
+    const int tid = threadIdx.x, wave = tid >> 6;
+    const int group = (int)xcd_group(gridDim.x);
+    if (group >= groups) return;
+    const int64_t r = (int64_t)group * kGroupThreads + tid;
+    const uint32_t g = (r < n) ? perm[r] : 0u;
+    const RankLane L = rect_lane(g, (r < n) ? drects[r] : make_uint2(0u, 0u));
+    group_masks(L, bg, s.row[wave], s.col[wave]);
+    const uint64_t below = lanemask_lt();
+    for (int s0 = 0; s0 < bg.nb; s0 += kGroupThreads) {
+        __syncthreads();
+        const int s1 = min(s0 + kGroupThreads, bg.nb);
+        if (s0 + tid < s1) {
+            const int b = s0 + tid, sy = b / bg.bw, sx = b - sy * bg.bw;
+            s_start[tid] = pos[(size_t)b * gstride + group];
+            uint32_t run = 0;
+#pragma unroll
+            for (int j = 0; j < kGroupChunks; ++j) {
+                s_rel[j][tid] = (uint16_t)run;
+                run += (uint32_t)popc64(s.row[j][sy] & s.col[j][sx]);
+            }
+        }
+        __syncthreads();
+        // the lane's blocks in the window's rows, one per step (no rows
+        // without a rectangle: bh is 0)
+        int sy = max(L.by0, s0 / bg.bw), sx = L.bx0;
+        const int y1 = min(L.by0 + (int)L.bh, (s1 - 1) / bg.bw + 1);
+        const int x1 = L.bx0 + (int)L.bw;
+        while (sy < y1) {
+            const int b = sy * bg.bw + sx;
+            if (b >= s0 && b < s1) {
+                const uint64_t p = (uint64_t)s_start[b - s0] + (uint64_t)s_rel[wave][b - s0] +
+                                   (uint64_t)popc64(s.row[wave][sy] & s.col[wave][sx] & below);
+                if (p < cap) {
+                    lists[p] = L.g;
+                    lrects[p] = local_rect(L.t, sx * 8, sy * 8);
+                }
+            }
+            const bool wrap = ++sx == x1;
+            sx = wrap ? L.bx0 : sx;
+            sy += wrap ? 1 : 0;
         }
     }
 }
@@ -487,7 +613,7 @@ __global__ __launch_bounds__(kThreads) void tile_scatter_kernel(
     const uint32_t nseg = min(uniform(seg_start[bg.nb]), seg_cap);
     const uint32_t stride = gridDim.x * kWavesPer;
     const int lane = lane_id();
-    for (uint32_t k = uniform(xcd_group() * kWavesPer + (threadIdx.x >> 6)); k < nseg;
+    for (uint32_t k = uniform(xcd_group(gridDim.x) * kWavesPer + (threadIdx.x >> 6)); k < nseg;
          k += stride) {
         const SegInfo I = seg_info(k, seg_owner, seg_start, block_start, bg.bw, bg.nb);
         const SegLane S = seg_lane<true>(lists, lrects, I.first, I.end, cap, n);
@@ -572,8 +698,8 @@ inline unsigned groups_for(uint64_t waves) {
 
 // Work-groups of the grid-strided segment kernels: enough for the bound on
 // segments, at most 8 per CU of a 256-CU device.
-// Pair lists beyond which tile_scatter runs fewer work-groups (1 GB of ids).
-constexpr uint64_t kScatterThrottlePairs = 1ull << 28;
+// Pair lists beyond which tile_scatter runs fewer work-groups (4 GB of ids).
+constexpr uint64_t kScatterThrottlePairs = 1ull << 30;
 
 inline unsigned seg_groups(uint64_t seg_bound) {
     return (unsigned)std::max<uint64_t>(1, std::min<uint64_t>(groups_for(seg_bound), 2048));
@@ -605,32 +731,55 @@ hipError_t launch_tile_binning(const TileBinning& tb, hipStream_t st) {
     if (tb.m == 0 || tb.n <= 0 || bg.nb <= 0) return hipSuccess;
     const int chunks = (int)(((size_t)tb.n + kWave - 1) / kWave);
     const int windows = (bg.nb + kWave - 1) / kWave;
-    const int cstride = (int)block_count_stride(tb.n);
     const uint64_t segs = segment_bound(tb.m, bg);
     if (segs > 0xffffffffull) return hipErrorInvalidValue;
     const uint32_t seg_cap = (uint32_t)segs;
     hipError_t e;
-    const uint64_t l1_waves = (uint64_t)chunks * (uint64_t)windows;
-    if (tb.drects) {
-        hipLaunchKernelGGL(rank_rects_kernel, dim3(groups_for(((uint64_t)tb.n + kWave - 1) / kWave)),
-                           dim3(kThreads), 0, st, tb.n, tb.perm, tb.rects, tb.drects);
-        if ((e = hipGetLastError()) != hipSuccess) return e;
-    }
     RecordArgs ra{tb.rec_mean2d, tb.rec_cov2d, tb.rec_colors, tb.rec_alpha,
-                  static_cast<BlendRec*>(tb.recs), groups_for(l1_waves)};
-    const unsigned rec_groups =
-        ra.recs ? (unsigned)(((size_t)tb.n + kThreads - 1) / kThreads) : 0u;
-    hipLaunchKernelGGL(block_count_kernel, dim3(ra.first + rec_groups), dim3(kThreads), 0, st,
-                       tb.n, tb.perm, tb.rects, tb.drects, bg, chunks, windows, cstride,
-                       tb.bcount, ra);
+                  static_cast<BlendRec*>(tb.recs), 0u};
+    // The grouped level 1 (its figures are at the kernels) from the count on at
+    // which the rectangles are gathered: at 100k Gaussians and 1080p its 196
+    // work-groups leave the chip idle, 30 us against 24.
+    const bool grouped = tb.drects && bg.bw <= kWave && bg.bh <= kWave;
+    const uint64_t l1_waves = (uint64_t)chunks * (uint64_t)windows;
+    const int groups = (int)(((size_t)tb.n + kGroupThreads - 1) / kGroupThreads);
+    const unsigned group_grid = ((unsigned)groups + 7u) / 8u * 8u;  // whole lists per XCD
+    const int l1_cols = grouped ? groups : chunks;
+    const int l1_stride = (l1_cols + 3) / 4 * 4;
+    if (grouped) {
+        ra.first = group_grid;
+        const unsigned rec_groups =
+            ra.recs ? (unsigned)(((size_t)tb.n + kGroupThreads - 1) / kGroupThreads) : 0u;
+        hipLaunchKernelGGL(group_count_kernel, dim3(group_grid + rec_groups), dim3(kGroupThreads),
+                           0, st, tb.n, tb.perm, tb.rects, tb.drects, bg, groups, l1_stride,
+                           tb.bcount, ra);
+    } else {
+        if (tb.drects) {
+            hipLaunchKernelGGL(rank_rects_kernel,
+                               dim3(groups_for(((uint64_t)tb.n + kWave - 1) / kWave)),
+                               dim3(kThreads), 0, st, tb.n, tb.perm, tb.rects, tb.drects);
+            if ((e = hipGetLastError()) != hipSuccess) return e;
+        }
+        ra.first = groups_for(l1_waves);
+        const unsigned rec_groups =
+            ra.recs ? (unsigned)(((size_t)tb.n + kThreads - 1) / kThreads) : 0u;
+        hipLaunchKernelGGL(block_count_kernel, dim3(ra.first + rec_groups), dim3(kThreads), 0, st,
+                           tb.n, tb.perm, tb.rects, tb.drects, bg, chunks, windows, l1_stride,
+                           tb.bcount, ra);
+    }
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    hipLaunchKernelGGL(block_scan_kernel, dim3(bg.nb), dim3(kThreads), 0, st, chunks, cstride,
+    hipLaunchKernelGGL(block_scan_kernel, dim3(bg.nb), dim3(kThreads), 0, st, l1_cols, l1_stride,
                        tb.bcount, tb.block_hist, tb.block_start, tb.seg_start, tb.seg_owner,
                        seg_cap, tb.err);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    hipLaunchKernelGGL(block_scatter_kernel, dim3(groups_for(l1_waves)), dim3(kThreads), 0, st,
-                       tb.n, tb.perm, tb.rects, tb.drects, bg, chunks, windows, cstride, tb.bcount,
-                       tb.lists, tb.lrects, tb.m);
+    if (grouped)
+        hipLaunchKernelGGL(group_scatter_kernel, dim3(group_grid), dim3(kGroupThreads), 0, st,
+                           tb.n, tb.perm, tb.drects, bg, groups, l1_stride, tb.bcount, tb.lists,
+                           tb.lrects, tb.m);
+    else
+        hipLaunchKernelGGL(block_scatter_kernel, dim3(groups_for(l1_waves)), dim3(kThreads), 0,
+                           st, tb.n, tb.perm, tb.rects, tb.drects, bg, chunks, windows, l1_stride,
+                           tb.bcount, tb.lists, tb.lrects, tb.m);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     hipLaunchKernelGGL(tile_count_kernel, dim3(seg_groups(segs)), dim3(kThreads), 0, st, tb.n, bg,
                        tb.seg_owner, tb.seg_start, tb.block_start, tb.lists, tb.m, tb.lrects,
@@ -643,13 +792,14 @@ hipError_t launch_tile_binning(const TileBinning& tb, hipStream_t st) {
                        bg.tiles_x * bg.tiles_y, tb.ttotal, tb.m,
                        reinterpret_cast<int2*>(tb.ranges), tb.err, tb.skip != nullptr);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    // Each wave writes its segment's 64 runs to 64 lists.  Once the lists
-    // are gigabytes (config c5: 7.4 GB per band, runs of ~13 ids), fewer
-    // waves in flight write faster: 2 work-groups per CU took c5's binning
-    // from 24.3 to 21.7 ms per frame, while 8 stay best at c4 (166 MB of ids:
-    // 166 us against 194) and at 1080p.
-    const unsigned scatter_groups =
-        tb.m > kScatterThrottlePairs ? std::min(seg_groups(segs), 512u) : seg_groups(segs);
+    // Each wave writes its segment's 64 runs to 64 lists.  Six work-groups per
+    // CU write fastest: 2.4 GB of ids in 974 us (at 2, 4 and 8 per CU 1056, 964
+    // and 997), two passes of needles with 2.0 GB in 992 us (1339, 1056, 1009);
+    // 8 per CU are no better at 166 MB.  Beyond 4 GB of ids two per CU do (six
+    // bands of 7.4 GB: 16.9 ms against 17.1).  With skipped tiles m is only a
+    // bound, far above what is written.
+    const bool throttle = tb.m > kScatterThrottlePairs && !tb.skip;
+    const unsigned scatter_groups = std::min(seg_groups(segs), throttle ? 512u : 1536u);
     hipLaunchKernelGGL(tile_scatter_kernel, dim3(scatter_groups), dim3(kThreads), 0, st, tb.n,
                        bg, tb.seg_owner, tb.seg_start, tb.block_start, tb.lists, tb.m, tb.lrects,
                        seg_cap, tb.tcount, reinterpret_cast<const int2*>(tb.ranges), tb.m,
