@@ -1086,14 +1086,12 @@ __device__ __forceinline__ float row_sum(float x) {
 // few hundred slots or fewer, 64 (one word) beyond, where claimed slots are
 // sparse and a row then covers 1024 slots per step.
 template <int kReduceRowLanes, int kGroup>
-__global__ __launch_bounds__(256) void pair_grad_reduce_kernel(
-    int n, GradSlots gs, float* __restrict__ dmean, float* __restrict__ dcov,
-    float* __restrict__ dcol, float* __restrict__ dalpha) {
+__device__ __forceinline__ void reduce_row(int n, int g, const GradSlots& gs,
+                                           float* __restrict__ dmean, float* __restrict__ dcov,
+                                           float* __restrict__ dcol, float* __restrict__ dalpha) {
     static_assert(kReduceRowLanes == 16 || kReduceRowLanes == 8, "rows of 16 or 8 lanes");
     static_assert(kGroup == 8 || kGroup == 64, "flag groups of 8 or 64 slots");
-    constexpr int kReduceGaussiansPerBlock = 256 / kReduceRowLanes;
     const int sub = threadIdx.x & (kReduceRowLanes - 1);
-    const int g = blockIdx.x * kReduceGaussiansPerBlock + (int)(threadIdx.x / kReduceRowLanes);
     // the flag bits of slots [grp, grp + kGroup), grp a multiple of kGroup
     // (the flag array is 256-byte aligned and padded to 64-bit words)
     auto group_bits = [&](uint64_t grp) -> uint64_t {
@@ -1139,9 +1137,8 @@ __global__ __launch_bounds__(256) void pair_grad_reduce_kernel(
             bits = nbits;
         }
     }
-    // a Gaussian without claimed slots adds nothing (at 4K most Gaussians
-    // have none in a given screen band): its outputs are not read or written,
-    // and a wave without any skips the row sums
+    // a Gaussian without claimed slots adds nothing: its outputs are not read or
+    // written, and a wave without any skips the row sums
     const uint64_t wave_claims = ballot(claimed);
     if (wave_claims == 0ull) return;
     // every lane takes part in the row sums (rows past n add zeros)
@@ -1166,6 +1163,57 @@ __global__ __launch_bounds__(256) void pair_grad_reduce_kernel(
         dcol[3 * (size_t)g + 1] = k1 + t[6];
         dcol[3 * (size_t)g + 2] = k2 + t[7];
         dalpha[g] = a0 + t[8];
+    }
+}
+
+template <int kReduceRowLanes, int kGroup>
+__global__ __launch_bounds__(256) void pair_grad_reduce_kernel(
+    int n, GradSlots gs, float* __restrict__ dmean, float* __restrict__ dcov,
+    float* __restrict__ dcol, float* __restrict__ dalpha) {
+    const int g = blockIdx.x * (256 / kReduceRowLanes) + (int)(threadIdx.x / kReduceRowLanes);
+    reduce_row<kReduceRowLanes, kGroup>(n, g, gs, dmean, dcov, dcol, dalpha);
+}
+
+// The same sums where claimed slots are few: each wave looks through the claim
+// bits of 16 Gaussians, four lanes and four words at a time, and only those with
+// a claimed slot get a row.  In a 4K frame of 5M Gaussians (112 slots each, most
+// behind opaque ones) a row per Gaussian spent 430 us almost wholly on loading
+// bits that are zero; here 193 us.
+constexpr int kSparseGaussians = 16;  // per wave
+
+template <int kGroup>
+__global__ __launch_bounds__(256) void pair_grad_reduce_sparse_kernel(
+    int n, GradSlots gs, float* __restrict__ dmean, float* __restrict__ dcov,
+    float* __restrict__ dcol, float* __restrict__ dalpha) {
+    const int lane = lane_id();
+    const int g0 = (int)(blockIdx.x * 4u + (threadIdx.x >> 6)) * kSparseGaussians;
+    const int i = g0 + (lane >> 2);
+    bool any = false;
+    if (i < n) {
+        const uint64_t base = gs.goff[i];
+        const uint64_t end = min(base + (uint64_t)gs.counts[i], gs.slots);
+        const uint64_t* words = reinterpret_cast<const uint64_t*>(gs.flags);
+        for (uint64_t w = (base >> 6) + (uint64_t)(lane & 3); w << 6 < end; w += 4) {
+            uint64_t bits = words[w];
+            if (w << 6 < base) bits &= ~0ull << (base - (w << 6));
+            if (end - (w << 6) < 64u) bits &= ~(~0ull << (end - (w << 6)));
+            any |= bits != 0;
+        }
+    }
+    // bit 4 j: Gaussian g0 + j has a claimed slot
+    uint64_t claimed = ballot(any);
+    claimed |= claimed >> 1;
+    claimed |= claimed >> 2;
+    claimed &= 0x1111111111111111ull;
+    while (claimed) {
+        // the next four, one per 16-lane row
+        int g = n;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            if (claimed && (lane >> 4) == r) g = g0 + (int)(__builtin_ctzll(claimed) >> 2);
+            claimed &= claimed - 1;
+        }
+        reduce_row<16, kGroup>(n, g, gs, dmean, dcov, dcol, dalpha);
     }
 }
 
@@ -1553,9 +1601,17 @@ hipError_t launch_pair_grad_reduce(int n, const GradSlots& gs, float* dmean, flo
                                    float* dcol, float* dalpha, hipStream_t st) {
     if (n <= 0) return hipSuccess;
     // 8-lane rows when a Gaussian averages at most 64 slots (one flag load per
-    // lane); word-sized flag groups beyond 256 slots per Gaussian
+    // lane); word-sized flag groups beyond 256 slots per Gaussian.  From 2^19
+    // Gaussians on, so many slots mean that most lie behind others: the sparse
+    // kernel, whose 16 Gaussians per wave still fill the chip (2^15 waves)
     if (gs.slots <= 64ull * (uint64_t)n)
         hipLaunchKernelGGL((pair_grad_reduce_kernel<8, 8>), dim3((unsigned)((n + 31) / 32)),
+                           dim3(256), 0, st, n, gs, dmean, dcov, dcol, dalpha);
+    else if (n >= (1 << 19) && gs.slots <= 256ull * (uint64_t)n)
+        hipLaunchKernelGGL((pair_grad_reduce_sparse_kernel<8>), dim3((unsigned)((n + 63) / 64)),
+                           dim3(256), 0, st, n, gs, dmean, dcov, dcol, dalpha);
+    else if (n >= (1 << 19))
+        hipLaunchKernelGGL((pair_grad_reduce_sparse_kernel<64>), dim3((unsigned)((n + 63) / 64)),
                            dim3(256), 0, st, n, gs, dmean, dcov, dcol, dalpha);
     else if (gs.slots <= 256ull * (uint64_t)n)
         hipLaunchKernelGGL((pair_grad_reduce_kernel<16, 8>), dim3((unsigned)((n + 15) / 16)),
