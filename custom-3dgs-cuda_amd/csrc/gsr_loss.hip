@@ -81,13 +81,42 @@ __device__ __forceinline__ bool interior(int y, int x, int H, int W) {
     return y >= kWinR && y < H - kWinR && x >= kWinR && x < W - kWinR;
 }
 
-// Adds input i's share, w[i - j] v, to the values j of a run it lies in.
+// 1 / b for b in [C1, 4]: the hardware's (1 ulp) corrected once by its exact
+// residual, a division's 0.5 ulp.
+__device__ __forceinline__ float reciprocal(float b) {
+    const float r = __builtin_amdgcn_rcpf(b);
+    return __builtin_fmaf(__builtin_fmaf(-b, r, 1.0f), r, r);
+}
+
+// Adds input i's share, w[i - j] v, to the values j of a run it lies in: the
+// vertical passes take the rows as their loads arrive.
 template <int kRun>
 __device__ __forceinline__ void run_add(float (&m)[kRun], const Window& win, int i, float v) {
 #pragma clang fp contract(fast)
 #pragma unroll
     for (int j = 0; j < kRun; ++j)
         if (i - j >= 0 && i - j < kWinTaps) m[j] += win.w[i - j] * v;
+}
+
+// The kRun neighbouring window sums of kRun + 10 values, each from the window's
+// ends inwards: the large middle taps come last, so most additions round a small
+// sum.  The horizontal passes, whose values lie in LDS, take them so.  In the
+// order of the taps dL/dimg was 1.78e-6 from 64 bits at 1920x1080, where the
+// horizontal pass first and a product w x times x per window had left 1.76e-6
+// (x^2 formed once leaves its rounding in every window it lies in); so it is
+// 1.42e-6, in the same time (62 and 47 us).  The vertical passes so as well gave
+// 1.15e-6, but waited for the last row first: 63.5 and 48.3 us.
+template <int kRun>
+__device__ __forceinline__ void run_sums(float (&m)[kRun], const Window& win,
+                                         const float (&v)[kRun + kWinTaps - 1]) {
+#pragma clang fp contract(fast)
+#pragma unroll
+    for (int k = 0; k < kWinTaps; ++k) {
+        const int tap = (k & 1) ? kWinTaps - 1 - k / 2 : k / 2;
+#pragma unroll
+        for (int j = 0; j < kRun; ++j)
+            m[j] = k == 0 ? win.w[tap] * v[j + tap] : m[j] + win.w[tap] * v[j + tap];
+    }
 }
 
 // The element at byte offset `at` of row y of a plane of interleaved pixels, 0
@@ -164,11 +193,14 @@ __attribute__((amdgpu_waves_per_eu(5))) void ssim_fwd_kernel(
     {
         const int r = tid / kRowRuns, u = tid - r * kRowRuns, grp = u / 3, ch = u - 3 * grp;
         const int c = 3 * kRunH * grp + ch;  // the run's first window and input column
-        float m[5][kRunH] = {};
+        float m[5][kRunH];
 #pragma unroll
-        for (int i = 0; i < kRunHIn; ++i)
+        for (int k = 0; k < 5; ++k) {
+            float v[kRunHIn];
 #pragma unroll
-            for (int k = 0; k < 5; ++k) run_add(m[k], win, i, s_v[k][r][c + 3 * i]);
+            for (int i = 0; i < kRunHIn; ++i) v[i] = s_v[k][r][c + 3 * i];
+            run_sums(m[k], win, v);
+        }
         const int gy = y0 + r;
 #pragma unroll
         for (int j = 0; j < kRunH; ++j) {
@@ -182,11 +214,8 @@ __attribute__((amdgpu_waves_per_eu(5))) void ssim_fwd_kernel(
             const float sxy = m[4][j] - mux * muy;
             const float a1 = 2.0f * mux * muy + kC1, a2 = 2.0f * sxy + kC2;
             const float b1 = mux * mux + muy * muy + kC1, b2 = sxx + syy + kC2;
-            // one reciprocal for 1 / b1, 1 / b2 and their product (b1 b2 is at
-            // least C1 C2 = 9e-8): the hardware's, corrected once by its residual
-            const float bb = b1 * b2, r0 = __builtin_amdgcn_rcpf(bb);
-            const float inv = r0 + r0 * (1.0f - bb * r0);
-            const float rb1 = b2 * inv, rb2 = b1 * inv;
+            const float rb1 = reciprocal(b1), rb2 = reciprocal(b2);
+            const float inv = rb1 * rb2;
             const float s = a1 * a2 * inv;
             ssum += window ? s : 0.0f;
             if (gmaps) {
@@ -291,11 +320,14 @@ __global__ __launch_bounds__(kLossThreads) void ssim_bwd_kernel(
     }
     __syncthreads();
     const int c = 3 * kRunH * grp + ch;
-    float m[3][kRunH] = {};
+    float m[3][kRunH];
 #pragma unroll
-    for (int i = 0; i < kRunHIn; ++i)
+    for (int k = 0; k < 3; ++k) {
+        float v[kRunHIn];
 #pragma unroll
-        for (int k = 0; k < 3; ++k) run_add(m[k], win, i, s_v[k][r][c + 3 * i]);
+        for (int i = 0; i < kRunHIn; ++i) v[i] = s_v[k][r][c + 3 * i];
+        run_sums(m[k], win, v);
+    }
 #pragma unroll
     for (int j = 0; j < kRunH; ++j) {
         if (gy >= H || gx + j >= W) continue;
