@@ -7,8 +7,7 @@
 // per-pixel share of the batch loads and of the backward's wave reductions;
 // more waves per tile shorten the longest tile's critical path.  A batch of
 // one list entry per thread is staged in LDS as 48 B blend records (one
-// coalesced record load per entry); lanes walk the batch with broadcast LDS
-// reads.  The forward's per-pixel arithmetic is the reference's, operation
+// record load per entry); lanes walk the batch with broadcast LDS reads.  The forward's per-pixel arithmetic is the reference's, operation
 // for operation (rasterize.cu:241-270); the backward's decisions are too
 // (rasterize_backward.cu:113-200).
 //
@@ -24,7 +23,8 @@
 // when none of its pixels is live; the tile stops when all are done.
 // Backward: the tile walks only entries [0, max n_contrib) of its list, back
 // to front (the reference walks all K entries and skips the tail per pixel),
-// and each wave skips entries beyond its own max n_contrib.  It takes its
+// and each wave skips entries beyond its own max n_contrib.  A batch holds only
+// entries that a strip meets (fill_batch).  A wave takes its
 // entries four at a time: their decisions in straight-line code, their colours'
 // products with dL/dpixel by matrix instructions, and their nine gradient sums
 // over the wave through one transposition in LDS (see group_sums).  The two
@@ -171,26 +171,18 @@ __device__ __forceinline__ BlendRec load_record(const BlendRec* __restrict__ rec
     return r;
 }
 
-// A staged entry: the record's a and b words, and of c the blue channel and the
-// strip bits (c.y is a.w / 2, exactly; qthr has served).
+// A staged entry of the forward: the record's a and b words, and of c the blue
+// channel and the strip bits (c.y is a.w / 2, exactly; qthr has served).
 template <int kPix>
 __device__ __forceinline__ void stage_entry(const BlendRec* __restrict__ recs, int g, int n,
                                             int tile, int tiles_x, float4* s_a, float4* s_b,
-                                            float2* s_c, int* s_id, int slot) {
+                                            float2* s_c, int slot) {
     const BlendRec r = load_record(recs, g, n);
     const bool ok = g >= 0 && g < n;
     s_a[slot] = r.a;
     s_b[slot] = r.b;
     const uint32_t bits = ok ? strip_bits<kPix>(r, tile, tiles_x) : 0u;
     s_c[slot] = make_float2(r.c.x, __uint_as_float(bits));
-    if (s_id) s_id[slot] = ok ? g : -1;
-}
-
-// The entry past a batch's last place, which fills up a backward group: its
-// opacity is 0, so no pixel blends it.
-__device__ __forceinline__ void stage_none(float4* s_a, float4* s_b, float2* s_c, int slot) {
-    s_a[slot] = s_b[slot] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    s_c[slot] = make_float2(0.0f, __uint_as_float(kPlainBit));
 }
 
 // Forward pixel state.  A pixel is done once a blend takes T below 1e-4
@@ -330,7 +322,7 @@ __global__ __launch_bounds__(Layout<kPix>::kThreads) void blend_fwd_kernel(
         const int g = next_id;
         __syncthreads();
         if (tid < cnt)
-            stage_entry<kPix>(recs, g, n, tile, tiles_x, s_a, s_b, s_c, nullptr, tid);
+            stage_entry<kPix>(recs, g, n, tile, tiles_x, s_a, s_b, s_c, tid);
         if (b0 + kBatch + tid < end) next_id = ids[b0 + kBatch + tid];
         __syncthreads();
         if (ballot(any_live(p)) != 0) {
@@ -441,11 +433,11 @@ __device__ __forceinline__ uint64_t decide_fast(float power, float o, uint64_t w
 }
 
 // One pixel's gradient step for a decided entry (rasterize_backward.cu:
-// 141-198); cg is the entry's colour . dL/dpixel.  A skipped entry enters with ae = 0, which leaves T (x / 1) and
-// accg unchanged and gives zero terms.  dL/dpower is alpha T (colour .
-// dL/dpixel less what lies behind); the caller zeroes it where alpha is
-// clamped.  This arithmetic only has to meet
-// the fp32 gradient tolerance and may use fused multiply-adds.
+// 141-198); cg is the entry's colour . dL/dpixel.  A skipped entry enters with
+// ae = 0, which leaves T (x / 1) and accg unchanged and gives zero terms.
+// dL/dpower is alpha T (colour . dL/dpixel less what lies behind); the caller
+// zeroes it where alpha is clamped.  This arithmetic only has to meet the fp32
+// gradient tolerance and may use fused multiply-adds.
 __device__ __forceinline__ BwdTerms bwd_update(BwdPixel& p, float ae, float cg) {
 #pragma clang fp contract(fast)
     BwdTerms t;
@@ -511,9 +503,10 @@ __device__ __forceinline__ BwdPixel load_bwd_pixel(bool in, int px, int py, int 
 //   them in LDS, the dpw pairs and then the alpha T pairs;
 // - each is read back transposed, lane 4b + j taking entry j's terms of the
 //   four lanes of quad b (four columns, two rows);
-// - it sums the quad's dpw moments about entry j's mean: about a centre shared by the entries a matrix product could
-//   form them, but where little beyond one pixel beside the mean blends, e^2
-//   would be the difference of numbers thousands of times its size;
+// - it sums the quad's dpw moments about entry j's mean: about a centre shared by
+//   the entries a matrix product could form them, but where little beyond one
+//   pixel beside the mean blends, e^2 would be the difference of numbers
+//   thousands of times its size;
 // - the colours' weights dL/dpixel are no entry's own, so their products are
 //   matrix instructions (v_mfma_f32_4x4x1, fp32: sixteen 4x4 outer products,
 //   one per quad, accumulated over the quad's eight pixels);
@@ -660,38 +653,186 @@ constexpr int kSplitNum = 37, kSplitDen = 100;
 // Most tiles split per backward launch (the launch has this many extra groups).
 constexpr int kSplitMax = 256;
 
-// The entries of one 64-entry chunk of a staged batch [lo, lo + cnt) that a wave
-// walks: those within its largest n_contrib whose strip bit is set, back to
-// front, as byte offsets of their places in s_a; filled up with the none entry
-// to a whole number of groups.  One ballot and one store per wave: the walk then
-// finds its entries without scalar work.
-struct ChunkList {
-    int count;
-    bool plain;   // all of them are
-    bool within;  // all of them lie within every pixel's n_contrib
-};
+// A batch of the backward in LDS: list entries that some strip of the tile meets
+// within its n_contrib, back to front, and per wave the list of those it walks:
+// the byte offsets of their places in `a` (the flag kListExact in the low bits),
+// filled up with the none entry to a whole number of groups.
 template <int kPix, int kBatch>
-__device__ __forceinline__ ChunkList chunk_list(const float2* s_c, int c0, int cnt, int lo,
-                                                int wave_last, uint32_t my_bit,
-                                                const int (&last)[kPix], int* list) {
-    const int l = lane_id();
-    const int e = c0 + l;
-    const bool in = e < cnt;
-    const uint32_t b = in ? __float_as_uint(s_c[min(e, kBatch - 1)].y) : 0u;
-    const uint64_t walk = ballot(in && lo + e + 1 <= wave_last && (b & my_bit) != 0u);
-    const uint64_t plain = ballot((b & kPlainBit) != 0u);
-    const int end = (min(c0 + kWave, cnt) - 1) * (int)sizeof(float4);
-    bool beyond = false;
-#pragma unroll
-    for (int k = 0; k < kPix; ++k) beyond |= last[k] < end;
-    ChunkList c{popc64(walk), (walk & ~plain) == 0, ballot(beyond) == 0};
-    if ((walk >> l) & 1u) list[popc64(l == 63 ? 0ull : walk >> (l + 1))] = e * (int)sizeof(float4);
-    if (l < kGroup - 1) list[c.count + l] = kBatch * (int)sizeof(float4);
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    return c;
+struct BwdBatch {
+    static constexpr int kWaves = Layout<kPix>::kWaves;
+    // one place more than the batch: the none entry, whose opacity is 0, so
+    // that no pixel blends it
+    float4 a[kBatch + 1];   // the record's a and b words
+    float4 b[kBatch + 1];
+    float blue[kBatch + 1];
+    float rho[kBatch + 1];  // ridge_slope
+    int id[kBatch];
+    __attribute__((aligned(16))) int list[kWaves][kBatch + kGroup];
+    // two windows' ballots: per wave of the entries its threads hold, those that
+    // each strip meets
+    uint64_t met[2][kWaves][kWaves];
+};
+constexpr int kListExact = 1;  // not a plain entry
+constexpr int kListFlags = 15;
+
+template <int kPix, int kBatch>
+__device__ __forceinline__ void stage_none(BwdBatch<kPix, kBatch>& s) {
+    s.a[kBatch] = s.b[kBatch] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    s.blue[kBatch] = s.rho[kBatch] = 0.0f;
 }
-constexpr int kListSize = kWave + kGroup;
+
+// The tile's list as the backward fills its batches from it, back to front:
+// positions [lo, hi) are left, next_id is thread t's id of position hi - 1 - t
+// (-1: none).
+struct BwdSource {
+    const int32_t* ids;  // of the tile's first entry
+    const BlendRec* recs;
+    int n, tile, tiles_x;
+    int lo, hi, next_id;
+    int width;        // entries of the next window
+    uint32_t window;  // windows taken so far
+    __device__ __forceinline__ int id_below(int p, int t) const {
+        return p - 1 - t >= lo ? ids[p - 1 - t] : -1;
+    }
+};
+
+// Fills the batch from the list, a window of 128 entries (or 64, below) at a
+// time, one per thread: each forms its entry's strip bits, and only entries with
+// one are staged, in order, until the batch is at least half full or the list
+// ends; what does not fit stays for the next batch.  So the barriers, the partial
+// sums and their flush are paid for entries that are walked, and groups fill up
+// across the windows: of a needle-shaped cloud's entries 4% meet a strip, of
+// uniform clouds' 45%.  Staging 64 or 128 list entries as they came, with groups
+// within 64 of them (1.57 places per entry of the needles), and so (same run):
+// blend_bwd 3.67 and 2.42 ms (5M needles, 4K), 254 and 248 us (1M Gaussians,
+// 1080p), 179 and 174 us (100k), 118 and 115 us (720p).
+// The 64-entry batch takes windows of 64 while more than 3/4 of them meet a
+// strip: of 128 half would be looked at twice (the benchmark frame, of whose
+// entries 85% do, 200 us so and 196).
+// strip_last: each strip's largest n_contrib; least_last: the least of this
+// wave's pixels.  Returns how many entries are staged; `first`: per pixel the
+// byte offset of the first of them within its n_contrib; `listed`: those that this
+// wave walks, and whether all of them are plain.  All threads of the work-group,
+// whose reads of the batch before end at its first barrier.
+template <int kPix, int kBatch>
+__device__ __forceinline__ int fill_batch(BwdBatch<kPix, kBatch>& s, BwdSource& src,
+                                          const int (&strip_last)[Layout<kPix>::kWaves],
+                                          int least_last, const BwdPixel (&px)[kPix],
+                                          int (&first)[kPix], int& listed, bool& plain) {
+    constexpr int kWaves = Layout<kPix>::kWaves, kThreads = Layout<kPix>::kThreads;
+    static_assert(kBatch <= kThreads, "an empty batch takes at least one entry of a window");
+    const int tid = (int)threadIdx.x, lane = lane_id();
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int count = 0, in_list[kWaves] = {};
+#pragma unroll
+    for (int k = 0; k < kPix; ++k) first[k] = 0;
+    do {
+        const int width = src.width, hi = src.hi;
+        const int g = tid < width ? src.next_id : -1;
+        const int p = hi - 1 - tid;
+        // the window below, if this one fits
+        src.next_id = src.id_below(hi - width, tid);
+        const BlendRec r = load_record(src.recs, g, src.n);
+        uint32_t bits = (g >= 0 && g < src.n) ? strip_bits<kPix>(r, src.tile, src.tiles_x) : 0u;
+        uint64_t met[kWaves][kWaves];  // [threads' wave][strip]
+        uint64_t* out = s.met[src.window & 1u][wave];
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) {
+            if (p >= strip_last[w]) bits &= ~(1u << w);
+            const uint64_t m = ballot(((bits >> w) & 1u) != 0u);
+            if (lane == 0) out[w] = m;
+        }
+        __syncthreads();
+        uint64_t any[kWaves];
+        int total = 0;
+#pragma unroll
+        for (int v = 0; v < kWaves; ++v) {
+            any[v] = 0;
+#pragma unroll
+            for (int w = 0; w < kWaves; ++w) {
+                met[v][w] = uniform64(s.met[src.window & 1u][v][w]);
+                any[v] |= met[v][w];
+            }
+            total += popc64(any[v]);
+        }
+        ++src.window;
+        if (count + total > kBatch) {
+            // the first entry that does not fit, and all after it, stay
+            int room = kBatch - count, taken = 0;
+#pragma unroll
+            for (int v = 0; v < kWaves; ++v) {
+                const int here = popc64(any[v]);
+                if (room >= 0 && here > room) {
+                    const uint64_t first = ballot(((any[v] >> lane) & 1u) != 0u &&
+                                                  popc_below(any[v]) == room);
+                    taken = v * kWave + (int)__builtin_ctzll(first);
+                    any[v] &= (first - 1);
+                    room = -1;
+                } else if (room < 0) {
+                    any[v] = 0;
+                } else {
+                    room -= here;
+                }
+            }
+            src.hi -= taken;
+            src.next_id = src.id_below(src.hi, tid);
+        } else {
+            src.hi -= min(width, hi - src.lo);
+        }
+        if constexpr (kBatch < kThreads) src.width = 4 * total > 3 * width ? kBatch : kThreads;
+        if (hi > least_last) {  // some pixel's n_contrib ends in or below the window
+#pragma unroll
+            for (int k = 0; k < kPix; ++k) {
+#pragma unroll
+                for (int v = 0; v < kWaves; ++v) {
+                    const int c = min(hi - px[k].last - v * kWave, kWave);
+                    first[k] += c > 0 ? popc64(any[v] << (kWave - c)) : 0;
+                }
+            }
+        }
+        int before = count;
+#pragma unroll
+        for (int v = 0; v < kWaves; ++v) {
+            if (v == wave && ((any[v] >> lane) & 1u) != 0u) {
+                const int slot = before + popc_below(any[v]);
+                s.a[slot] = r.a;
+                s.b[slot] = r.b;
+                s.blue[slot] = r.c.x;
+                s.rho[slot] = ridge_slope(r.a);
+                s.id[slot] = g;
+                const int entry =
+                    slot * (int)sizeof(float4) | ((bits & kPlainBit) ? 0 : kListExact);
+#pragma unroll
+                for (int w = 0; w < kWaves; ++w)
+                    if ((bits >> w) & 1u)
+                        s.list[w][in_list[w] + popc_below(met[v][w] & any[v])] = entry;
+            }
+            before += popc64(any[v]);
+#pragma unroll
+            for (int w = 0; w < kWaves; ++w) in_list[w] += popc64(met[v][w] & any[v]);
+        }
+        count = before;
+    } while (count < kBatch / 2 && src.hi > src.lo);
+#pragma unroll
+    for (int k = 0; k < kPix; ++k) first[k] *= (int)sizeof(float4);
+    listed = 0;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) listed = w == wave ? in_list[w] : listed;
+    if (lane < kGroup - 1) s.list[wave][listed + lane] = kBatch * (int)sizeof(float4);
+    __syncthreads();
+    int flags = 0;
+    for (int e = lane; e < listed; e += kWave) flags |= s.list[wave][e];
+    plain = ballot((flags & kListFlags) != 0) == 0;
+    return count;
+}
+
+template <int kPix>
+__device__ __forceinline__ bool all_within(const int (&first)[kPix]) {
+    int some = 0;
+#pragma unroll
+    for (int k = 0; k < kPix; ++k) some |= first[k];
+    return ballot(some != 0) == 0;
+}
 
 template <typename T>
 __device__ __forceinline__ T staged(const void* base, int offset) {
@@ -702,11 +843,11 @@ __device__ __forceinline__ T staged(const void* base, int offset) {
 // the entries' colours (lane l reads entry l & 3's, at `own`) by the lanes' own
 // dL/dpixel, as three outer products per pixel (v_mfma_f32_4x4x1; lane l keeps
 // its pixel's column).
-template <int kPix>
-__device__ __forceinline__ void group_colours(int own, const float4* s_b, const float2* s_c,
+template <int kPix, int kBatch>
+__device__ __forceinline__ void group_colours(int own, const BwdBatch<kPix, kBatch>& st,
                                               const BwdPixel (&p)[kPix], f32x4 (&cg)[kPix]) {
-    const float2 rg = staged<float2>(s_b, own + (int)sizeof(float2));
-    const float b = staged<float>(s_c, own / 2);
+    const float2 rg = staged<float2>(st.b, own + (int)sizeof(float2));
+    const float b = staged<float>(st.blue, own / 4);
 #pragma unroll
     for (int k = 0; k < kPix; ++k) {
         f32x4 c = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -719,8 +860,8 @@ __device__ __forceinline__ void group_colours(int own, const float4* s_b, const 
 // The wave's decisions for a group's entries, all of them in straight-line code
 // (independent chains, one test for the whole group): the fast evaluation, then
 // the exact one for the whole wave for every entry that is not plain or has a
-// lane near the threshold.  at: the entries' offsets; last: the offset of the
-// last entry of the batch that each pixel blends.
+// lane near the threshold.  at: the group's part of the wave's list; within: the
+// whole batch lies within every pixel's n_contrib.
 template <int kPix>
 struct GroupDecision {
     float ae[kGroup][kPix];
@@ -732,29 +873,37 @@ __device__ __forceinline__ float staged_power(const float4& A, float c, float fx
     const float dx = fx - A.x, dy = fy - A.y;
     return __builtin_fmaf(c * dy, dy, __builtin_fmaf(A.w * dx, dy, (A.z * dx) * dx));
 }
-template <int kPix>
-__device__ __forceinline__ void decide_group(GroupDecision<kPix>& d, const int4& at,
-                                             const ChunkList& cl, float fx, const float (&fy)[kPix],
-                                             const int (&last)[kPix], const float4* s_a,
-                                             const float4* s_b, const float2* s_c) {
-    const int off[kGroup] = {at.x, at.y, at.z, at.w};
+template <int kPix, int kBatch>
+__device__ __forceinline__ void decide_group(GroupDecision<kPix>& d, const int4& at, bool plain, bool within,
+                                             const int (&first)[kPix], float fx,
+                                             const float (&fy)[kPix], const BwdBatch<kPix, kBatch>& st) {
+    int off[kGroup] = {at.x, at.y, at.z, at.w};
+    bool exact[kGroup] = {};
+    if (!plain) {
+#pragma unroll
+        for (int s = 0; s < kGroup; ++s) {
+            exact[s] = (__builtin_amdgcn_readfirstlane(off[s]) & kListExact) != 0;
+            off[s] &= ~kListFlags;
+        }
+    }
     float4 A[kGroup];
     float2 B[kGroup];
 #pragma unroll
     for (int s = 0; s < kGroup; ++s) {
-        A[s] = staged<float4>(s_a, off[s]);
-        B[s] = staged<float2>(s_b, off[s]);
+        A[s] = staged<float4>(st.a, off[s]);
+        B[s] = staged<float2>(st.b, off[s]);
     }
-    uint64_t within[kGroup][kPix];
+    uint64_t in[kGroup][kPix];
 #pragma unroll
     for (int s = 0; s < kGroup; ++s)
 #pragma unroll
-        for (int k = 0; k < kPix; ++k) within[s][k] = ~0ull;
-    if (!cl.within) {
+        for (int k = 0; k < kPix; ++k) in[s][k] = ~0ull;
+    if (!within) {
 #pragma unroll
-        for (int s = 0; s < kGroup; ++s)
+        for (int s = 0; s < kGroup; ++s) {
 #pragma unroll
-            for (int k = 0; k < kPix; ++k) within[s][k] = ballot(off[s] <= last[k]);
+            for (int k = 0; k < kPix; ++k) in[s][k] = ballot(off[s] >= first[k]);
+        }
     }
     uint64_t act = 0, odd[kGroup], odd_any = 0;
 #pragma unroll
@@ -762,24 +911,22 @@ __device__ __forceinline__ void decide_group(GroupDecision<kPix>& d, const int4&
         odd[s] = 0;
 #pragma unroll
         for (int k = 0; k < kPix; ++k) {
-            act |= decide_fast(staged_power(A[s], B[s].x, fx, fy[k]), B[s].y, within[s][k],
+            act |= decide_fast(staged_power(A[s], B[s].x, fx, fy[k]), B[s].y, in[s][k],
                                d.ae[s][k], odd[s]);
             d.clamped[s][k] = 0;
         }
         odd_any |= odd[s];
     }
     uint64_t clamped = 0;
-    if (odd_any != 0 || !cl.plain) {
+    if (odd_any != 0 || !plain) {
 #pragma unroll
         for (int s = 0; s < kGroup; ++s) {
-            const uint32_t bits = (uint32_t)__builtin_amdgcn_readfirstlane(
-                (int)staged<uint32_t>(s_c, off[s] / 2 + (int)sizeof(float)));
-            if (odd[s] == 0 && (bits & kPlainBit) != 0) continue;
-            const float4 a = staged<float4>(s_a, off[s]);
-            const float2 b = staged<float2>(s_b, off[s]);
+            if (odd[s] == 0 && !exact[s]) continue;
+            const float4 a = staged<float4>(st.a, off[s]);
+            const float2 b = staged<float2>(st.b, off[s]);
 #pragma unroll
             for (int k = 0; k < kPix; ++k) {
-                act |= decide_exact(staged_power(a, b.x, fx, fy[k]), b.y, within[s][k],
+                act |= decide_exact(staged_power(a, b.x, fx, fy[k]), b.y, in[s][k],
                                     d.ae[s][k], d.clamped[s][k]);
                 clamped |= d.clamped[s][k];
             }
@@ -791,51 +938,30 @@ __device__ __forceinline__ void decide_group(GroupDecision<kPix>& d, const int4&
     d.any_clamped = clamped != 0;
 }
 
-// Per pixel the offset of the last entry of the batch at list position lo that
-// it blends (negative: none).
+// The pixel state's walk over the source's entries: the same decisions and T /
+// accumulated-colour steps as the full walk, no sums.
 template <int kPix, int kBatch>
-__device__ __forceinline__ void last_offsets(const BwdPixel (&p)[kPix], int lo,
-                                             int (&last)[kPix]) {
+__device__ __forceinline__ void state_walk(BwdSource src,
+                                           const int (&strip_last)[Layout<kPix>::kWaves],
+                                           int least_last, float fx, const float (&fy)[kPix],
+                                           BwdPixel (&p)[kPix], BwdBatch<kPix, kBatch>& st) {
+    const int* list = st.list[__builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6)];
+    while (src.hi > src.lo) {
+        int listed, first[kPix];
+        bool plain;
+        if (fill_batch(st, src, strip_last, least_last, p, first, listed, plain) == 0) break;
+        const bool within = all_within(first);
+        for (int i = 0; i < listed; i += kGroup) {
+            const int4 at = *reinterpret_cast<const int4*>(list + i);
+            GroupDecision<kPix> d;
+            decide_group(d, at, plain, within, first, fx, fy, st);
+            if (!d.any) continue;  // as the full walk
+            f32x4 cg[kPix];
+            group_colours(list[i + (lane_id() & 3)] & ~kListFlags, st, p, cg);
 #pragma unroll
-    for (int k = 0; k < kPix; ++k)
-        last[k] = min(max(p[k].last - lo - 1, -1), kBatch - 1) * (int)sizeof(float4);
-}
-
-// The pixel state's walk over entries [lo0, hi0), back to front: the same
-// decisions and T / accumulated-colour steps as the full walk, no sums.
-template <int kPix, int kBatch>
-__device__ __forceinline__ void state_walk(int lo0, int hi0, int n, int tile, int tiles_x,
-                                           int start, int wave_last, uint32_t my_bit, float fx,
-                                           const float (&fy)[kPix], BwdPixel (&p)[kPix],
-                                           const int32_t* __restrict__ ids,
-                                           const BlendRec* __restrict__ recs, float4* s_a,
-                                           float4* s_b, float2* s_c, int* list) {
-    const int tid = threadIdx.x;
-    for (int hi = hi0; hi > lo0; hi -= kBatch) {
-        const int lo = max(lo0, hi - kBatch);
-        const int cnt = hi - lo;
-        __syncthreads();
-        if (tid < cnt)
-            stage_entry<kPix>(recs, ids[start + lo + tid], n, tile, tiles_x, s_a, s_b, s_c,
-                              nullptr, tid);
-        __syncthreads();
-        int last[kPix];
-        last_offsets<kPix, kBatch>(p, lo, last);
-        for (int chunk = ((cnt - 1) / kWave) * kWave; chunk >= 0; chunk -= kWave) {
-            const ChunkList cl = chunk_list<kPix, kBatch>(s_c, chunk, cnt, lo, wave_last, my_bit,
-                                                          last, list);
-            for (int i = 0; i < cl.count; i += kGroup) {
-                const int4 at = *reinterpret_cast<const int4*>(list + i);
-                GroupDecision<kPix> d;
-                decide_group<kPix>(d, at, cl, fx, fy, last, s_a, s_b, s_c);
-                if (!d.any) continue;  // as the full walk
-                f32x4 cg[kPix];
-                group_colours<kPix>(list[i + (lane_id() & 3)], s_b, s_c, p, cg);
+            for (int s = 0; s < kGroup; ++s) {
 #pragma unroll
-                for (int s = 0; s < kGroup; ++s) {
-#pragma unroll
-                    for (int k = 0; k < kPix; ++k) (void)bwd_update(p[k], d.ae[s][k], cg[k][s]);
-                }
+                for (int k = 0; k < kPix; ++k) (void)bwd_update(p[k], d.ae[s][k], cg[k][s]);
             }
         }
     }
@@ -851,18 +977,11 @@ __attribute__((amdgpu_waves_per_eu(kBatch == 64 ? 6 : 4))) void blend_bwd_kernel
     float* __restrict__ dcol, float* __restrict__ dalpha, GradSlots gs,
     const uint32_t* __restrict__ order) {
     constexpr int kWaves = Layout<kPix>::kWaves;
-    static_assert(kBatch <= Layout<kPix>::kThreads, "one staged entry per thread");
-    // one place more than the batch: the none entry (stage_none)
-    __shared__ float4 s_a[kBatch + 1];
-    __shared__ float4 s_b[kBatch + 1];
-    __shared__ float2 s_c[kBatch + 1];
-    __shared__ float s_rho[kBatch + 1];
-    __shared__ int s_id[kBatch];
+    __shared__ BwdBatch<kPix, kBatch> st;
     // +1: the none entry, and a group's writers hit different banks
     __shared__ float s_part[kWaves][kTerms][kBatch + 1];
-    __shared__ __attribute__((aligned(16))) int s_list[kWaves][kListSize];
     __shared__ float2 s_terms[kWaves][kGroup * kGroupPitch];
-    __shared__ uint32_t s_max[kWaves];
+    __shared__ int s_max[kWaves];
 
     // Work item.  kSplit (a schedule is given): items 2i and 2i + 1 (i < K) are
     // the back and front parts of the schedule's i-th tile, and the later
@@ -889,115 +1008,102 @@ __attribute__((amdgpu_waves_per_eu(kBatch == 64 ? 6 : 4))) void blend_bwd_kernel
     if ((unsigned)tile >= (unsigned)T) return;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // scalar: uniform branches
-    const uint32_t my_bit = 1u << wave;
     static_assert(kPix == 2, "group_sums takes two pixels per lane");
     const Pixels<kPix> pp = bwd_pixels_of(tile, tiles_x, W, H);
     const int tx = tile % tiles_x, ty = tile / tiles_x;
     const float fx = (float)pp.px;
     float fy[kPix];
     BwdPixel p[kPix];
-    int my_last = 0;
+    int my_last = 0, my_least = 0x7fffffff;
 #pragma unroll
     for (int k = 0; k < kPix; ++k) {
         fy[k] = (float)pp.py[k];
         p[k] = load_bwd_pixel(pp.in[k], pp.px, pp.py[k], W, grad, gst, finalT, ncontrib);
         my_last = max(my_last, p[k].last);
+        my_least = min(my_least, p[k].last);
     }
     int start, end;
     clamp_range(ranges[tile], m, start, end);
     const int wave_last = __builtin_amdgcn_readfirstlane((int)wave_max_u32((uint32_t)my_last));
-    if (lane == 0) s_max[wave] = (uint32_t)wave_last;
+    const int least_last = 0x7fffffff - __builtin_amdgcn_readfirstlane(
+        (int)wave_max_u32(0x7fffffffu - (uint32_t)my_least));
+    if (lane == 0) s_max[wave] = wave_last;
     __syncthreads();
-    uint32_t tile_last = 0;
+    int strip_last[kWaves], tile_last = 0;
 #pragma unroll
-    for (int w = 0; w < kWaves; ++w) tile_last = max(tile_last, s_max[w]);
-    const int maxc = __builtin_amdgcn_readfirstlane(min((int)tile_last, end - start));
+    for (int w = 0; w < kWaves; ++w) {
+        strip_last[w] = __builtin_amdgcn_readfirstlane(s_max[w]);
+        tile_last = max(tile_last, strip_last[w]);
+    }
     start = __builtin_amdgcn_readfirstlane(start);
+    const int maxc = min(tile_last, __builtin_amdgcn_readfirstlane(end) - start);
     const int my_value = group_value_of_lane(lane);
     const GroupWeights wt = group_weights(p);
     const float x0 = (float)(tx * kTileSize + (lane & 12));  // the quad's first column
-    int* list = s_list[wave];
-    if (tid == 0) {  // before the first batch's barriers
-        stage_none(s_a, s_b, s_c, kBatch);
-        s_rho[kBatch] = 0.0f;
-    }
+    if (tid == 0) stage_none(st);  // before the first batch's barriers
     float2* terms = s_terms[wave];
-    // the entries [lo0, hi0) this item walks with gradients; the front part
-    // first walks [mid, maxc) for the pixel state only
-    int lo0 = 0, hi0 = maxc;
+    const int* list = st.list[wave];
+    // the entries [lo, hi) this item walks with gradients; the front part first
+    // walks [mid, maxc) for the pixel state only
+    BwdSource src{ids + start, recs, n, tile, tiles_x, 0, maxc, -1, kBatch, 0u};
     if constexpr (kSplit) {
         const int mid = (int)(((int64_t)maxc * kSplitNum) / kSplitDen);
-        if (part == kPartBack) lo0 = mid;
+        if (part == kPartBack) src.lo = mid;
         if (part == kPartFront) {
-            hi0 = mid;
-            state_walk<kPix, kBatch>(mid, maxc, n, tile, tiles_x, start, wave_last, my_bit, fx,
-                                     fy, p, ids, recs, s_a, s_b, s_c, list);
+            BwdSource behind = src;
+            behind.lo = mid;
+            behind.next_id = behind.id_below(maxc, tid);
+            state_walk(behind, strip_last, least_last, fx, fy, p, st);
+            src.hi = mid;
         }
     }
 
-    // each batch's ids are loaded while the batch after it is walked
-    int next_id =
-        (tid < min(hi0 - lo0, kBatch)) ? ids[start + max(lo0, hi0 - kBatch) + tid] : -1;
-    for (int hi = hi0; hi > lo0; hi -= kBatch) {
-        const int lo = max(lo0, hi - kBatch);
-        const int cnt = hi - lo;
-        const int g = next_id;
-        // the staging's and the flush's addresses are formed again per batch:
-        // kept through the walk they cost it registers, then scratch
+    src.next_id = src.id_below(src.hi, tid);
+    while (src.hi > src.lo) {
+        // the flush's addresses are formed again per batch: kept through the
+        // walk they cost it registers, then scratch
         int tid = (int)threadIdx.x;
         asm volatile("" : "+v"(tid));
-        __syncthreads();
-        if (tid < cnt) {
-            stage_entry<kPix>(recs, g, n, tile, tiles_x, s_a, s_b, s_c, s_id, tid);
-            s_rho[tid] = ridge_slope(s_a[tid]);
-        }
-        if (lo > lo0) {
-            const int nlo = max(lo0, lo - kBatch);
-            if (tid < lo - nlo) next_id = ids[start + nlo + tid];
-        }
-        __syncthreads();
+        int listed, first[kPix];
+        bool plain;
+        const int cnt = fill_batch(st, src, strip_last, least_last, p, first, listed, plain);
+        if (cnt == 0) break;
         // this wave's partial sums of the batch start at zero: entries it does
-        // not walk (culled, or beyond its largest n_contrib) add nothing
+        // not walk add nothing
         for (int e = lane; e < cnt; e += kWave)
 #pragma unroll
             for (int k = 0; k < kTerms; ++k) s_part[wave][k][e] = 0.0f;
-        int last[kPix];
-        last_offsets<kPix, kBatch>(p, lo, last);
-        for (int chunk = ((cnt - 1) / kWave) * kWave; chunk >= 0; chunk -= kWave) {
-            const ChunkList cl = chunk_list<kPix, kBatch>(s_c, chunk, cnt, lo, wave_last, my_bit,
-                                                          last, list);
-            for (int i = 0; i < cl.count; i += kGroup) {
-                const int4 at = *reinterpret_cast<const int4*>(list + i);
-                const int own = list[i + (lane & 3)];
-                GroupDecision<kPix> d;
-                decide_group<kPix>(d, at, cl, fx, fy, last, s_a, s_b, s_c);
-                // no pixel blends an entry: the state stays and the sums are zero
-                if (!d.any) continue;
-                f32x4 cg[kPix];
-                group_colours<kPix>(own, s_b, s_c, p, cg);
-                BwdTerms q[kGroup][kPix];
+        const bool within = all_within(first);
+        for (int i = 0; i < listed; i += kGroup) {
+            const int4 at = *reinterpret_cast<const int4*>(list + i);
+            const int own = list[i + (lane & 3)] & ~kListFlags;
+            GroupDecision<kPix> d;
+            decide_group(d, at, plain, within, first, fx, fy, st);
+            // no pixel blends an entry: the state stays and the sums are zero
+            if (!d.any) continue;
+            f32x4 cg[kPix];
+            group_colours(own, st, p, cg);
+            BwdTerms q[kGroup][kPix];
+#pragma unroll
+            for (int s = 0; s < kGroup; ++s)
+#pragma unroll
+                for (int k = 0; k < kPix; ++k)
+                    q[s][k] = bwd_update(p[k], d.ae[s][k], cg[k][s]);
+            if (d.any_clamped) {
 #pragma unroll
                 for (int s = 0; s < kGroup; ++s)
 #pragma unroll
                     for (int k = 0; k < kPix; ++k)
-                        q[s][k] = bwd_update(p[k], d.ae[s][k], cg[k][s]);
-                if (d.any_clamped) {
-#pragma unroll
-                    for (int s = 0; s < kGroup; ++s)
-#pragma unroll
-                        for (int k = 0; k < kPix; ++k)
-                            if (__builtin_amdgcn_inverse_ballot_w64(d.clamped[s][k]))
-                                q[s][k].dpw = 0.0f;
-                }
-                const float sum =
-                    group_sums(terms, wt, q, x0, fy, staged<float2>(s_a, own),
-                               staged<float>(s_rho, own / 4));
-                if (my_value >= 0) s_part[wave][my_value][own / (int)sizeof(float4)] = sum;
+                        if (__builtin_amdgcn_inverse_ballot_w64(d.clamped[s][k]))
+                            q[s][k].dpw = 0.0f;
             }
+            const float sum = group_sums(terms, wt, q, x0, fy, staged<float2>(st.a, own),
+                                         staged<float>(st.rho, own / 4));
+            if (my_value >= 0) s_part[wave][my_value][own / (int)sizeof(float4)] = sum;
         }
         __syncthreads();
         if (tid < cnt) {
-            const int g = s_id[tid];
+            const int g = st.id[tid];
             float tot[kTerms];
             bool any = false;
 #pragma unroll
@@ -1008,11 +1114,11 @@ __attribute__((amdgpu_waves_per_eu(kBatch == 64 ? 6 : 4))) void blend_bwd_kernel
                 tot[k] = acc;
                 any |= acc != 0.0f;
             }
-            if (g >= 0 && any) {
+            if (any) {
                 float t[kTerms];
                 // the record's -cx/2 (A.z), -cy (A.w), -cz/2 (B.x), opacity (B.y)
-                const float cx = -2.0f * s_a[tid].z, cy = -s_a[tid].w, cz = -2.0f * s_b[tid].x;
-                const float o = s_b[tid].y, rho = s_rho[tid];
+                const float cx = -2.0f * st.a[tid].z, cy = -st.a[tid].w, cz = -2.0f * st.b[tid].x;
+                const float o = st.b[tid].y, rho = st.rho[tid];
                 const float r = __builtin_fmaf(-cx, rho, cy), k = __builtin_fmaf(-cy, rho, cz);
                 const float S0 = tot[kS0], P1 = tot[kP1], P2 = tot[kP2];
                 const float Q1 = tot[kQ1], Q2 = tot[kQ2], P5 = tot[kP5];

@@ -119,6 +119,18 @@ __device__ __forceinline__ uint64_t lanemask_lt() {
 
 __device__ __forceinline__ int popc64(uint64_t m) { return __builtin_popcountll(m); }
 
+// Set bits of m in lanes strictly below this one.
+__device__ __forceinline__ int popc_below(uint64_t m) {
+    return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+                                          __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+}
+
+// A value that is the same in all lanes, as a scalar.
+__device__ __forceinline__ uint64_t uniform64(uint64_t v) {
+    return (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v) |
+           (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32)) << 32;
+}
+
 // Adds one to LDS histogram bin d for every active lane.  A wave whose active
 // lanes all have the same bin adds their count once: a bin hit by whole waves
 // (a byte every key shares) would otherwise take 64 same-address atomics per
