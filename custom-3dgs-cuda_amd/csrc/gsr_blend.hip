@@ -119,19 +119,18 @@ __device__ __forceinline__ float qmin_rect(float mx, float my, float A, float B,
     return best;
 }
 
-// Staged strip bits: bit w for wave w of the tile, and this flag for a plain
-// entry: a plain record (plain_record) whose quadratic form's |terms| sum to at
-// most kPlainTerms over the tile, so that exp's argument reduction holds and
-// gives 0 or a denormal far below the range, an alpha below 1/255 either way.
-constexpr uint32_t kPlainBit = 1u << 31;
+// Staged strip bits: bit w for wave w of the tile, and the record's flags
+// (plain_record) where its quadratic form's |terms| sum to at most kPlainTerms over
+// the tile, so that exp's argument reduction holds and gives 0 or a denormal far
+// below the range, an alpha below 1/255 either way.
 constexpr float kPlainTerms = 4e6f;
 
 // Bit w set: some pixel of strip w may reach alpha >= 1/255.  A strip is
 // culled when the least q over its rectangle, lowered by 1e-5 of the largest
 // sum of |terms| there (the fp32 rounding of the per-pixel q and of this
 // bound are each within ~1e-6 of that sum), still exceeds qthr.  Conics that
-// are not positive definite, and NaN anywhere, cull nothing.  With kPlainBit
-// for a plain entry.
+// are not positive definite, and NaN anywhere, cull nothing.  With the
+// flags of a plain entry.
 template <int kPix>
 __device__ __forceinline__ uint32_t strip_bits(const BlendRec& r, int tile, int tiles_x) {
     constexpr uint32_t kAll = (1u << Layout<kPix>::kWaves) - 1u;
@@ -156,7 +155,7 @@ __device__ __forceinline__ uint32_t strip_bits(const BlendRec& r, int tile, int 
         bits |= skip ? 0u : (1u << w);
         most = (absq <= most) ? most : absq;  // NaN stays
     }
-    return bits | (r.c.w == kPlainRecord && most <= kPlainTerms ? kPlainBit : 0u);
+    return bits | (most <= kPlainTerms ? __float_as_uint(r.c.w) : 0u);
 }
 
 // The record of list entry g, zeros for an id outside [0, n) (such entries are
@@ -224,20 +223,23 @@ __device__ __forceinline__ void fwd_step(FwdPixel& p, bool on, float fx, float f
     p.last = blend ? contributor : p.last;
 }
 
-// fwd_step of the next kCount plain entries (kPlainBit) of `todo` in list order,
-// bit for bit: a plain entry's power is never positive, its alpha never clamped,
-// exp needs no range select, and one select of alpha serves the colours and T
-// (a weight of 0 adds nothing, T times 1 is T): 28 VALU per pixel and entry
-// instead of 35.  The alphas do not depend on T: all of the group's are formed
-// first, in straight-line code with independent chains, then blended in order.
+// fwd_step of the next kCount plain entries (kPlainBit, or kClampBit with `clamp`;
+// no kColourBit) of `todo` in list order, bit for bit: a plain entry's power is
+// never positive, its alpha never clamped (else with `clamp`, one minimum), exp
+// needs no range select, and one select of alpha serves the colours and T (a
+// weight of 0 adds nothing, T times 1 is T): 28 VALU per pixel and entry instead of
+// 35.  The alphas do not depend on T: all of the group's are formed first, in
+// straight-line code with independent chains, then blended in order.
 // Measured with a step per entry and so (same run): 140 and 123 us (100k
-// Gaussians, 1080p), 180 and 157 us (1M), 48 and 41 us (10k, 256x256).
+// Gaussians, 1080p), 180 and 157 us (1M), 48 and 41 us (10k, 256x256).  Where
+// 64 entries held one of an opacity from 0.99 on, all took fwd_step; frames with
+// half of the opacities there, and now: 426 and 418 us (1080p), 269 and 259 us.
 constexpr int kFwdGroup = 4;
 template <int kPix, int kCount>
 __device__ __forceinline__ void fwd_steps_plain(FwdPixel (&p)[kPix], float fx,
                                                 const float (&fy)[kPix], const float4* s_a,
                                                 const float4* s_b, const float2* s_c, int c0,
-                                                uint64_t& todo, int cbase) {
+                                                uint64_t& todo, int cbase, bool clamp) {
     float alpha[kCount][kPix];
     int at[kCount];
 #pragma unroll
@@ -255,6 +257,12 @@ __device__ __forceinline__ void fwd_steps_plain(FwdPixel (&p)[kPix], float fx,
             const float a = B.y * exp_core(power);
             alpha[s][k] = (a < kAlphaMin) ? 0.0f : a;
         }
+    }
+    if (clamp) {
+#pragma unroll
+        for (int s = 0; s < kCount; ++s)
+#pragma unroll
+            for (int k = 0; k < kPix; ++k) alpha[s][k] = fminf(kAlphaMax, alpha[s][k]);
     }
 #pragma unroll
     for (int s = 0; s < kCount; ++s) {
@@ -335,16 +343,18 @@ __global__ __launch_bounds__(Layout<kPix>::kThreads) void blend_fwd_kernel(
                 const int e = c0 + lane;
                 const uint32_t bits = e < cnt ? __float_as_uint(s_c[min(e, kBatch - 1)].y) : 0u;
                 uint64_t todo = ballot((bits & my_bit) != 0u);
-                const uint64_t plain = ballot((bits & kPlainBit) != 0u);
+                const uint64_t odd =
+                    todo & ballot((bits & (kPlainBit | kClampBit)) == 0u || (bits & kColourBit));
+                const bool clamp = (todo & ballot((bits & kClampBit) != 0u)) != 0;
                 // the wave stops once no pixel is live, tested before each group
                 // or entry with the same compares the steps' skips use
-                if ((todo & ~plain) == 0) {
+                if (odd == 0) {
                     int left = popc64(todo);
                     for (; left >= kFwdGroup && ballot(any_live(p)) != 0; left -= kFwdGroup)
                         fwd_steps_plain<kPix, kFwdGroup>(p, fx, fy, s_a, s_b, s_c, c0, todo,
-                                                         cbase);
+                                                         cbase, clamp);
                     for (; left > 0 && ballot(any_live(p)) != 0; --left)
-                        fwd_steps_plain<kPix, 1>(p, fx, fy, s_a, s_b, s_c, c0, todo, cbase);
+                        fwd_steps_plain<kPix, 1>(p, fx, fy, s_a, s_b, s_c, c0, todo, cbase, clamp);
                 } else {
                     while (todo && ballot(any_live(p)) != 0) {
                         const int j = c0 + (int)__builtin_ctzll(todo);
@@ -399,16 +409,14 @@ struct BwdTerms {
 // the lanes that blend it.
 //
 // The forward's own evaluation: exp_blend and the same fp32 operations, so
-// every skip agrees with the forward bit for bit.  `clamped`: the lanes whose
-// alpha is clamped (no gradient through alpha).
+// every skip agrees with the forward bit for bit.
 __device__ __forceinline__ uint64_t decide_exact(float power, float o, uint64_t within,
-                                                 float& ae, uint64_t& clamped) {
+                                                 float& ae) {
     const float araw = o * exp_blend(power);
     const float alpha = fminf(kAlphaMax, araw);
     const uint64_t act =
         within & ballot(!(power > 0.0f)) & ballot(!(alpha < kAlphaMin));
     ae = __builtin_amdgcn_inverse_ballot_w64(act) ? alpha : 0.0f;
-    clamped = act & ~ballot(araw < kAlphaMax);
     return act;
 }
 
@@ -865,8 +873,8 @@ __device__ __forceinline__ void group_colours(int own, const BwdBatch<kPix, kBat
 template <int kPix>
 struct GroupDecision {
     float ae[kGroup][kPix];
-    uint64_t clamped[kGroup][kPix];
-    bool any, any_clamped;  // some pixel blends an entry, some alpha is clamped
+    bool any;      // some pixel blends an entry
+    bool clamped;  // an alpha may be clamped: it is then kAlphaMax itself, and only then
 };
 __device__ __forceinline__ float staged_power(const float4& A, float c, float fx, float fy) {
     // the forward's power, bit for bit (blend_power)
@@ -874,9 +882,10 @@ __device__ __forceinline__ float staged_power(const float4& A, float c, float fx
     return __builtin_fmaf(c * dy, dy, __builtin_fmaf(A.w * dx, dy, (A.z * dx) * dx));
 }
 template <int kPix, int kBatch>
-__device__ __forceinline__ void decide_group(GroupDecision<kPix>& d, const int4& at, bool plain, bool within,
-                                             const int (&first)[kPix], float fx,
-                                             const float (&fy)[kPix], const BwdBatch<kPix, kBatch>& st) {
+__device__ __forceinline__ void decide_group(GroupDecision<kPix>& d, const int4& at, bool plain,
+                                             bool within, const int (&first)[kPix], float fx,
+                                             const float (&fy)[kPix],
+                                             const BwdBatch<kPix, kBatch>& st) {
     int off[kGroup] = {at.x, at.y, at.z, at.w};
     bool exact[kGroup] = {};
     if (!plain) {
@@ -910,32 +919,27 @@ __device__ __forceinline__ void decide_group(GroupDecision<kPix>& d, const int4&
     for (int s = 0; s < kGroup; ++s) {
         odd[s] = 0;
 #pragma unroll
-        for (int k = 0; k < kPix; ++k) {
+        for (int k = 0; k < kPix; ++k)
             act |= decide_fast(staged_power(A[s], B[s].x, fx, fy[k]), B[s].y, in[s][k],
                                d.ae[s][k], odd[s]);
-            d.clamped[s][k] = 0;
-        }
         odd_any |= odd[s];
     }
-    uint64_t clamped = 0;
+    d.clamped = false;
     if (odd_any != 0 || !plain) {
 #pragma unroll
         for (int s = 0; s < kGroup; ++s) {
             if (odd[s] == 0 && !exact[s]) continue;
+            d.clamped |= exact[s];
             const float4 a = staged<float4>(st.a, off[s]);
             const float2 b = staged<float2>(st.b, off[s]);
 #pragma unroll
-            for (int k = 0; k < kPix; ++k) {
-                act |= decide_exact(staged_power(a, b.x, fx, fy[k]), b.y, in[s][k],
-                                    d.ae[s][k], d.clamped[s][k]);
-                clamped |= d.clamped[s][k];
-            }
+            for (int k = 0; k < kPix; ++k)
+                act |= decide_exact(staged_power(a, b.x, fx, fy[k]), b.y, in[s][k], d.ae[s][k]);
         }
     }
     // act may hold an entry's fast decision that the exact one took back: the
     // group is then summed for nothing
     d.any = act != 0;
-    d.any_clamped = clamped != 0;
 }
 
 // The pixel state's walk over the source's entries: the same decisions and T /
@@ -1089,13 +1093,12 @@ __attribute__((amdgpu_waves_per_eu(kBatch == 64 ? 6 : 4))) void blend_bwd_kernel
 #pragma unroll
                 for (int k = 0; k < kPix; ++k)
                     q[s][k] = bwd_update(p[k], d.ae[s][k], cg[k][s]);
-            if (d.any_clamped) {
+            if (d.clamped) {
 #pragma unroll
                 for (int s = 0; s < kGroup; ++s)
 #pragma unroll
                     for (int k = 0; k < kPix; ++k)
-                        if (__builtin_amdgcn_inverse_ballot_w64(d.clamped[s][k]))
-                            q[s][k].dpw = 0.0f;
+                        q[s][k].dpw = d.ae[s][k] == kAlphaMax ? 0.0f : q[s][k].dpw;
             }
             const float sum = group_sums(terms, wt, q, x0, fy, staged<float2>(st.a, own),
                                          staged<float>(st.rho, own / 4));

@@ -268,8 +268,8 @@ constexpr uint32_t kSpinLimit = 1u << 22;
 // opacity, r, g), (b, -conic.y/2, qthr, plain).  The conic terms carry the
 // power's -1/2 (exact scalings by powers of two), so the blend evaluates
 // power = fma(c dy, dy, fma(b dx, dy, (a dx) dx)) without the final multiply;
-// the conic itself is -2 times them, exactly.  The last word is kPlainRecord
-// for a plain record (plain_record), else 0.
+// the conic itself is -2 times them, exactly.  The last word holds
+// the flags of a plain record (plain_record).
 // qthr bounds the quadratic form from above for any pixel that can reach
 // alpha >= 1/255 (conservative; negative when the opacity alone rules every
 // pixel out): the blends use it to skip entries for whole pixel regions
@@ -292,21 +292,26 @@ __device__ __forceinline__ float alpha_q_threshold(float o) {
 
 // A plain record, which both blends step without the tests that it cannot fail
 // (and with the bound on the power's terms that they add per tile):
-// - opacity in [0, 0.99): alpha = opacity G is never clamped, as G <= 1;
 // - a conic A, C >= 1e-12, B^2 <= (1 - 4e-5) A C: the power's terms sum to at
 //   most -1.9e-5 of (|a| dx^2 + |c| dy^2), forty times the sum of its roundings,
 //   so the computed power is never positive (the mean 0 or at least 1e-10 from
 //   0 per axis, so no product of an offset underflows);
-// - colours in [0, inf): a weight of 0 adds exactly nothing.
-// NaN anywhere makes a record not plain.
-constexpr float kPlainRecord = 1.0f;
-__device__ __forceinline__ bool plain_record(float mx, float my, float A, float B, float C,
-                                             float opacity, float r, float g, float b) {
+// - opacity in [0, 1]: kPlainBit below 0.99, where alpha = opacity G is never
+//   clamped, as G <= 1; kClampBit from 0.99 on, where it may be (a trained cloud
+//   holds many at its bound on the logit, an fp32 sigmoid of 0.99000007);
+// - kColourBit too for a colour outside [0, inf): with any other a weight of 0 adds
+//   exactly nothing.
+// 0 for any other record, and for NaN in the mean, conic or opacity.
+constexpr uint32_t kPlainBit = 1u << 29, kClampBit = 1u << 30, kColourBit = 1u << 31;
+__device__ __forceinline__ uint32_t plain_record(float mx, float my, float A, float B, float C,
+                                                 float opacity, float r, float g, float b) {
     auto away = [](float m) { return m == 0.0f || fabsf(m) >= 1e-10f; };
     auto colour = [](float c) { return c >= 0.0f && c < __builtin_inff(); };
-    return opacity >= 0.0f && opacity < kAlphaMax && A >= 1e-12f && C >= 1e-12f &&
-           B * B <= 0.99996f * (A * C) && away(mx) && away(my) && colour(r) && colour(g) &&
-           colour(b);
+    if (!(opacity >= 0.0f && opacity <= 1.0f && A >= 1e-12f && C >= 1e-12f &&
+          B * B <= 0.99996f * (A * C) && away(mx) && away(my)))
+        return 0u;
+    return (opacity < kAlphaMax ? kPlainBit : kClampBit) |
+           (colour(r) && colour(g) && colour(b) ? 0u : kColourBit);
 }
 
 // Conic = cov^-1 with 1/det first (rasterize.cu:224-232), packed with mean,
@@ -320,7 +325,7 @@ __device__ __forceinline__ BlendRec blend_record(float mx, float my, float a, fl
     rec.a = make_float4(mx, my, -0.5f * cx, -cy);
     rec.b = make_float4(-0.5f * cz, opacity, r, g);
     rec.c = make_float4(bl, -0.5f * cy, alpha_q_threshold(opacity),
-                        plain_record(mx, my, cx, cy, cz, opacity, r, g, bl) ? kPlainRecord : 0.0f);
+                        __uint_as_float(plain_record(mx, my, cx, cy, cz, opacity, r, g, bl)));
     return rec;
 }
 
