@@ -1175,9 +1175,6 @@ __attribute__((amdgpu_waves_per_eu(kBatch == 64 ? 6 : 4))) void blend_bwd_kernel
     }
 }
 
-// One 16-lane row per Gaussian (four per wave): the nine sums of its flagged
-// slots (d mean2d, d cov2d, d colour, d opacity), added to the outputs (which
-// hold zeros and any fallback atomics from the blend).
 // Sum over the kLanes (16 or 8) lanes of each row, result in every lane of
 // the row.
 template <int kLanes>
@@ -1189,7 +1186,10 @@ __device__ __forceinline__ float row_sum(float x) {
     return x;
 }
 
-// kLanes per Gaussian: 16, or 8 when Gaussians have few slots (half the
+// One row of lanes per Gaussian: the nine sums of its flagged
+// slots (d mean2d, d cov2d, d colour, d opacity), added to the outputs (which
+// hold zeros and any fallback atomics from the blend).
+// kReduceRowLanes per Gaussian: 16, or 8 when Gaussians have few slots (half the
 // waves then wait on the dependent loads).  Each lane reads the flag bits of
 // kGroup consecutive slots per step: 8 (one byte) when Gaussians average a
 // few hundred slots or fewer, 64 (one word) beyond, where claimed slots are
@@ -1286,8 +1286,8 @@ __global__ __launch_bounds__(256) void pair_grad_reduce_kernel(
 // The same sums where claimed slots are few: each wave looks through the claim
 // bits of 16 Gaussians, four lanes and four words at a time, and only those with
 // a claimed slot get a row.  In a 4K frame of 5M Gaussians (112 slots each, most
-// behind opaque ones) a row per Gaussian spent 430 us almost wholly on loading
-// bits that are zero; here 193 us.
+// behind opaque ones) a row per Gaussian spent 425 us almost wholly on loading
+// bits that are zero; here 174 us.  8 Gaussians per wave: 204.
 constexpr int kSparseGaussians = 16;  // per wave
 
 template <int kGroup>
@@ -1710,9 +1710,16 @@ hipError_t launch_pair_grad_reduce(int n, const GradSlots& gs, float* dmean, flo
                                    float* dcol, float* dalpha, hipStream_t st) {
     if (n <= 0) return hipSuccess;
     // 8-lane rows when a Gaussian averages at most 64 slots (one flag load per
-    // lane); word-sized flag groups beyond 256 slots per Gaussian.  From 2^19
-    // Gaussians on, so many slots mean that most lie behind others: the sparse
-    // kernel, whose 16 Gaussians per wave still fill the chip (2^15 waves)
+    // lane); word-sized flag groups beyond 256 slots per Gaussian.  Beyond 64
+    // slots, from 2^19 Gaussians on (2^15 waves of the sparse kernel, four times
+    // what the chip holds), a tile's list averages over 1000 entries at 4K: mostly
+    // they end behind what hides them, and the sparse kernel is the faster, 51
+    // against 72 us (600k Gaussians of 78 slots, opacity 0.5) and 174 against
+    // 425.  A cloud faint enough to be seen through is summed 5% slower, 284
+    // against 264 us (600k of opacity 0.02), 337 against 313 (0.05), 450 against
+    // 428 (540k wider ones), as its waves, four times as long, end less evenly:
+    // 0.2% of those frames (13 ms and more); which of them a frame is, only the
+    // blend knows.
     if (gs.slots <= 64ull * (uint64_t)n)
         hipLaunchKernelGGL((pair_grad_reduce_kernel<8, 8>), dim3((unsigned)((n + 31) / 32)),
                            dim3(256), 0, st, n, gs, dmean, dcov, dcol, dalpha);
