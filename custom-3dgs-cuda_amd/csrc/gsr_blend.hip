@@ -653,11 +653,12 @@ __device__ __forceinline__ float ridge_slope(const float4& A) {
 // pixel state only (state_walk) (the T and accumulated-colour steps of
 // rasterize_backward.cu:141-198, no gradient sums), which hands it the exact
 // state the sequential walk has at mid, then walks [0, mid) in full.  Both
-// parts' gradients are bit for bit the whole tile's.  A state-only step costs
-// about 0.4 of a full one, so mid = 0.37 maxc leaves each part ~0.63 of the
-// tile's walk.
+// parts' gradients are bit for bit the whole tile's.  mid = 0.30 maxc: the two
+// parts then take about as long (at 0.23, 0.27, 0.30, 0.37 and 0.44: 73.8, 73.1,
+// 72.6, 75.7 and 79.3 us, 10k Gaussians at 256x256; six bands of lists of 350k
+// entries 3.72, 3.77, 3.79, 3.84 and 3.88 ms; 720p between 121 and 124 us at all).
 constexpr int kPartWhole = 0, kPartBack = 1, kPartFront = 2;
-constexpr int kSplitNum = 37, kSplitDen = 100;
+constexpr int kSplitNum = 30, kSplitDen = 100;
 // Most tiles split per backward launch (the launch has this many extra groups).
 constexpr int kSplitMax = 256;
 
@@ -1585,8 +1586,9 @@ bool fwd_grid_fits(unsigned tiles) { return tiles <= device_facts().fwd_resident
 
 // Whether the backward's grid of tiles is resident on the device at once, or
 // so nearly (4/3 of what fits: 4096 tiles) that its longest tiles set its
-// length and the 128-entry batch with the split pays: 720p (3600 tiles) 121 us
-// so and 127 with 64-entry batches, 1080p (8160 tiles) 224 and 209.
+// length and the 128-entry batch with the split pays: 256x256 76 us so and 110
+// with 64-entry batches, 720p (3600 tiles) 122 and 127, 1080p (8160 tiles) 215 and
+// 214, with a million Gaussians 276 and 266.
 bool bwd_grid_fits(unsigned tiles) {
     return (uint64_t)tiles * 3 <= (uint64_t)device_facts().bwd_resident * 4;
 }
@@ -1594,9 +1596,10 @@ bool bwd_grid_fits(unsigned tiles) {
 // Lists that average this many entries per tile or more (the screen bands of
 // config c5 average ~350k) are walked like a resident grid's: 128-entry
 // batches with the longest tiles split.  Their longest tiles set the kernel's
-// length there (c5: blend_bwd 8.0 ms per frame with 64-entry batches, 5.5 with
-// 128, 4.5 with 128 and the split), while at 1080p (1.6k entries per tile) the
-// 64-entry batch without the split stays ahead (251 us against 259).
+// length there (blend_bwd 4.14 ms per frame with 64-entry batches, 3.84 so), while
+// the 64-entry batch without the split stays ahead at 1080p (1.6k entries per
+// tile) and for the 4K needles of the depth-prefix frame (11k): 266 us against
+// 276, 2.45 ms against 2.62.
 constexpr uint64_t kLongListAvg = 32768;
 bool bwd_long_lists(unsigned tiles, uint64_t pairs) {
     return pairs >= kLongListAvg * (uint64_t)tiles;
@@ -1687,8 +1690,8 @@ hipError_t launch_blend_bwd(int n, int H, int W, const float* grad, const GradSt
     // and the split's extra state-only walk costs more than it saves.
     const bool wide = bwd_wide(tiles, num_pairs);
     const bool split = order && bwd_split() && wide;
-    // The 64-entry batch takes 12.5 KB of LDS (13 work-groups per CU, as many
-    // as its registers allow); it pays when the grid does not fit on the device
+    // The 64-entry batch takes 12.3 KB of LDS and 80 registers (6 waves per SIMD,
+    // 12 work-groups per CU); it pays when the grid does not fit on the device
     // at once.  When it would, the 128-entry batch (20 KB) leaves part of the
     // grid to be placed as CUs free up, which balances the long tiles better.
     if (!wide)
