@@ -223,23 +223,23 @@ __device__ __forceinline__ void fwd_step(FwdPixel& p, bool on, float fx, float f
     p.last = blend ? contributor : p.last;
 }
 
-// fwd_step of the next kCount plain entries (kPlainBit, or kClampBit with `clamp`;
+// fwd_step of the next kCount plain entries (kPlainBit, or kClampBit with kClamp;
 // no kColourBit) of `todo` in list order, bit for bit: a plain entry's power is
-// never positive, its alpha never clamped (else with `clamp`, one minimum), exp
-// needs no range select, and one select of alpha serves the colours and T (a
-// weight of 0 adds nothing, T times 1 is T): 28 VALU per pixel and entry instead of
-// 35.  The alphas do not depend on T: all of the group's are formed first, in
-// straight-line code with independent chains, then blended in order.
+// never positive, its alpha never clamped (kClamp: one minimum), exp needs no range
+// select, and one select of alpha serves the colours and T (a weight of 0 adds
+// nothing, T times 1 is T): 28 VALU per pixel and entry instead of 35.  The alphas
+// do not depend on T: all of the group's are formed first, in straight-line code
+// with independent chains, then blended in order.
 // Measured with a step per entry and so (same run): 140 and 123 us (100k
-// Gaussians, 1080p), 180 and 157 us (1M), 48 and 41 us (10k, 256x256).  Where
-// 64 entries held one of an opacity from 0.99 on, all took fwd_step; frames with
-// half of the opacities there, and now: 426 and 418 us (1080p), 269 and 259 us.
+// Gaussians, 1080p), 180 and 157 us (1M), 48 and 41 us (10k, 256x256).  With half of the
+// opacities from 0.99 on, by fwd_step and so: 97 and 88 us (100k, 1080p), 53 and 43
+// us (10k, 256x256).
 constexpr int kFwdGroup = 4;
-template <int kPix, int kCount>
+template <int kPix, int kCount, bool kClamp>
 __device__ __forceinline__ void fwd_steps_plain(FwdPixel (&p)[kPix], float fx,
                                                 const float (&fy)[kPix], const float4* s_a,
                                                 const float4* s_b, const float2* s_c, int c0,
-                                                uint64_t& todo, int cbase, bool clamp) {
+                                                uint64_t& todo, int cbase) {
     float alpha[kCount][kPix];
     int at[kCount];
 #pragma unroll
@@ -254,15 +254,10 @@ __device__ __forceinline__ void fwd_steps_plain(FwdPixel (&p)[kPix], float fx,
         for (int k = 0; k < kPix; ++k) {
             const float dy = fy[k] - A.y;
             const float power = __builtin_fmaf(B.x * dy, dy, __builtin_fmaf(bdx, dy, adxdx));
-            const float a = B.y * exp_core(power);
+            float a = B.y * exp_core(power);
+            if constexpr (kClamp) a = fminf(kAlphaMax, a);
             alpha[s][k] = (a < kAlphaMin) ? 0.0f : a;
         }
-    }
-    if (clamp) {
-#pragma unroll
-        for (int s = 0; s < kCount; ++s)
-#pragma unroll
-            for (int k = 0; k < kPix; ++k) alpha[s][k] = fminf(kAlphaMax, alpha[s][k]);
     }
 #pragma unroll
     for (int s = 0; s < kCount; ++s) {
@@ -287,6 +282,22 @@ __device__ __forceinline__ bool any_live(const FwdPixel (&p)[kPix]) {
 #pragma unroll
     for (int k = 0; k < kPix; ++k) l |= live(p[k]);
     return l;
+}
+
+// Steps `todo`'s entries, all of them plain, while a pixel is live.
+template <int kPix, bool kClamp>
+__device__ __forceinline__ void fwd_walk_plain(FwdPixel (&p)[kPix], float fx,
+                                               const float (&fy)[kPix], const float4* s_a,
+                                               const float4* s_b, const float2* s_c, int c0,
+                                               uint64_t& todo, int cbase) {
+    // two at a time where four would take more registers than eight waves per SIMD
+    // leave (71 of 64)
+    constexpr int kCount = kClamp && kPix == 2 ? 2 : kFwdGroup;
+    int left = popc64(todo);
+    for (; left >= kCount && ballot(any_live(p)) != 0; left -= kCount)
+        fwd_steps_plain<kPix, kCount, kClamp>(p, fx, fy, s_a, s_b, s_c, c0, todo, cbase);
+    for (; left > 0 && ballot(any_live(p)) != 0; --left)
+        fwd_steps_plain<kPix, 1, kClamp>(p, fx, fy, s_a, s_b, s_c, c0, todo, cbase);
 }
 
 template <int kPix>
@@ -343,18 +354,14 @@ __global__ __launch_bounds__(Layout<kPix>::kThreads) void blend_fwd_kernel(
                 const int e = c0 + lane;
                 const uint32_t bits = e < cnt ? __float_as_uint(s_c[min(e, kBatch - 1)].y) : 0u;
                 uint64_t todo = ballot((bits & my_bit) != 0u);
-                const uint64_t odd =
-                    todo & ballot((bits & (kPlainBit | kClampBit)) == 0u || (bits & kColourBit));
-                const bool clamp = (todo & ballot((bits & kClampBit) != 0u)) != 0;
+                constexpr uint32_t kAny = kPlainBit | kClampBit | kColourBit;
+                const uint64_t odd = todo & ballot((bits & kAny) != kPlainBit);
                 // the wave stops once no pixel is live, tested before each group
                 // or entry with the same compares the steps' skips use
                 if (odd == 0) {
-                    int left = popc64(todo);
-                    for (; left >= kFwdGroup && ballot(any_live(p)) != 0; left -= kFwdGroup)
-                        fwd_steps_plain<kPix, kFwdGroup>(p, fx, fy, s_a, s_b, s_c, c0, todo,
-                                                         cbase, clamp);
-                    for (; left > 0 && ballot(any_live(p)) != 0; --left)
-                        fwd_steps_plain<kPix, 1>(p, fx, fy, s_a, s_b, s_c, c0, todo, cbase, clamp);
+                    fwd_walk_plain<kPix, false>(p, fx, fy, s_a, s_b, s_c, c0, todo, cbase);
+                } else if ((odd & ballot((bits & kAny) != kClampBit)) == 0) {
+                    fwd_walk_plain<kPix, true>(p, fx, fy, s_a, s_b, s_c, c0, todo, cbase);
                 } else {
                     while (todo && ballot(any_live(p)) != 0) {
                         const int j = c0 + (int)__builtin_ctzll(todo);
