@@ -157,6 +157,17 @@ def test_committed_profiles_were_measured_on_these_sources(monkeypatch, name):
         assert bench.stale_reason(prof, entry) is None, (key, bench.stale_reason(prof, entry))
 
 
+def test_c5_traffic_was_measured_on_these_sources(monkeypatch):
+    """The same for the 4K frames of 5M Gaussians, kept per kernel."""
+    prof = bench._profile_json("traffic", "c5_5M_3840x2160_banded")
+    assert prof and set(prof["sources"]) == set(_tree_sources())
+    monkeypatch.setattr(bench, "library_sources", _tree_sources)
+    own = {k: v["source_file"] for k, v in prof["kernels"].items() if v["source_file"]}
+    assert any(k.startswith("blend_bwd_kernel") for k in own)
+    for key, source in own.items():
+        assert bench.stale_reason(prof, {"source_files": [source]}) is None, key
+
+
 def _changed(name):
     out = dict(SOURCES)
     out[name] = "f" * 16
