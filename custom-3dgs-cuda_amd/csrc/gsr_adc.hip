@@ -199,10 +199,11 @@ struct KeptRows {
 // of dst, element-parallel over the destination: whole-line stores, loads
 // coalesced up to the dropped rows (cached: the rows left out share their lines,
 // and streaming stores of the short runs cost 30% more).  With `clamp` the value is
-// min(v, hi), NaN kept.  What bounds the pass is HBM (every parameter and moment
-// in once and out once: 1M sources with 12% new rows 311 us, 4.8 TB/s); with one
-// loop over the source elements and four destination lookups each it was VALU
-// issue and one chain of 18 arrays per work-group (519 us).
+// min(v, hi), NaN kept.  Every parameter and moment goes in once and out once: 1M
+// sources with 12% new rows 311 us, 4.8 TB/s, a device copy's rate, where the
+// optimizer's kernel, which leaves no rows out, reaches 5.6; with one loop over the
+// source elements and four destination lookups each it was VALU issue and one
+// chain of 18 arrays per work-group (519 us).
 template <int W>
 __device__ __forceinline__ void copy_list(const float* __restrict__ src, float* __restrict__ dst,
                                           const KeptRows& k, bool clamp = false,
